@@ -14,7 +14,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libmicpmd.so"
 
-HIP_SOURCES = ["context.hip", "wfft.hip", "gemm.hip", "gemm_x3.hip", "gemm_planes.hip", "ortho.hip", "vofrho.hip",
+HIP_SOURCES = ["context.hip", "wfft.hip", "gemm.hip", "gemm_f64.hip", "gemm_x3.hip", "gemm_planes.hip", "ortho.hip", "vofrho.hip",
                "capi.hip", "restart.hip", "probe.hip"]
 
 HIPCC_FLAGS = [

@@ -13,6 +13,11 @@
 //    (k x n) small; optional upper-triangular G (trmm) and a fused complex
 //    epilogue for fnonloc.
 //
+// Products of 16-byte aligned operands with even leading dimensions (all
+// wavefunction products; A G from 4096 rows) run in the kernels of
+// gemm_f64.hip; the ones here take what is left: small A G products and
+// operands of odd leading dimension or 8-byte alignment.
+//
 // Each workgroup computes a 128x128 tile (64x64 for small problems) with 4
 // waves (2x2), each wave a 64x64 block = 4x4 MFMA tiles of 16x16 (64 FP64
 // accumulators per lane).  Operands
@@ -179,77 +184,68 @@ __global__ __launch_bounds__(256) void k_gemm_tn(const double* __restrict__ A, i
     }
 }
 
-// out(i,j) = alpha * sum_s P[s](i,j) - g0 * a0(i) b0(j); symmetric: only the
-// upper triangle is used and mirrored into the lower one (dmatc).
-// out(i, j) = alpha sum_q P[q](i, j) [- A(0, i) B(0, j)], partials P[q] of
-// ldp rows (the first m used), mirrored from the upper triangle if symmetric
-// sum_q P[q * stride + o], q = 0 .. nsplit-1 in order; eight loads in flight
-// per step (the adds keep the sequential order, so the sum is the same)
-__device__ __forceinline__ double sum_partials(const double* __restrict__ P, int nsplit, size_t stride, size_t o) {
+// Sums of split-K partials.  A workgroup of 256 sums 32 consecutive elements of
+// one column: 8 groups of 32 lanes take a contiguous range of the splits each
+// (eight loads in flight per lane), and the group sums are added in order, so
+// the result does not depend on the launch.  With few columns and many splits
+// (128 states: 128 x 128 elements, 267 splits) this keeps hundreds of
+// workgroups busy where one per 32 x 32 block left 10 (47 -> 10 us).
+__device__ __forceinline__ double sum_partials(const double* __restrict__ P, int nsplit, size_t stride, size_t o,
+                                               bool on) {
+  __shared__ double part[8][32];
+  const int lane = threadIdx.x & 31, grp = threadIdx.x >> 5;
+  const int per = (nsplit + 7) / 8, q1 = min(nsplit, (grp + 1) * per);
   double s = 0.0;
-  int q = 0;
-  for (; q + 8 <= nsplit; q += 8) {
+  int q = on ? grp * per : q1;
+  for (; q + 8 <= q1; q += 8) {
     double v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) v[u] = P[(size_t)(q + u) * stride + o];
 #pragma unroll
     for (int u = 0; u < 8; ++u) s += v[u];
   }
-  for (; q < nsplit; ++q) s += P[(size_t)q * stride + o];
-  return s;
-}
-
-__global__ void k_reduce_tn(const double* __restrict__ P, int nsplit, int ldp, int m, int n, double alpha,
-                            const double* __restrict__ a0, int lda, const double* __restrict__ b0, int ldb,
-                            int g0, int symmetric, double* __restrict__ out, int ldo) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y;
-  if (i >= m || j >= n) return;
-  int si = i, sj = j;
-  if (symmetric && i > j) { si = j; sj = i; }
-  const double s = sum_partials(P, nsplit, (size_t)ldp * n, (size_t)sj * ldp + si);
-  double v = alpha * s;
-  if (g0) v -= a0[(size_t)si * lda] * b0[(size_t)sj * ldb];
-  out[(size_t)j * ldo + i] = v;
-}
-
-// The symmetric case of k_reduce_tn (m == n, only tiles on or above the
-// diagonal computed): out(i, j) = out(j, i) = the value of k_reduce_tn at
-// i <= j.  One workgroup per 32 x 32 block (bi <= bj): coalesced sums down the
-// columns of P, the mirrored block written through LDS.
-__global__ __launch_bounds__(256) void k_reduce_tn_sym(const double* __restrict__ P, int nsplit, int ldp, int n,
-                                                       double alpha, const double* __restrict__ a0, int lda,
-                                                       const double* __restrict__ b0, int ldb, int g0,
-                                                       double* __restrict__ out, int ldo) {
-  __shared__ double tile[32][33];
-  const int nb = (n + 31) / 32;
-  int bi = 0, bj = blockIdx.x;   // blockIdx.x -> (bi, bj), bi <= bj, row-major over the upper triangle
-  while (bj >= nb - bi) {
-    bj -= nb - bi;
-    ++bi;
-  }
-  bj += bi;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const int i = 32 * bi + tx;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int jl = ty + 8 * u, j = 32 * bj + jl;
-    double v = 0.0;
-    if (i < n && j < n && i <= j) {
-      const double s = sum_partials(P, nsplit, (size_t)ldp * n, (size_t)j * ldp + i);
-      v = alpha * s;
-      if (g0) v -= a0[(size_t)i * lda] * b0[(size_t)j * ldb];
-      out[(size_t)j * ldo + i] = v;
-    }
-    tile[tx][jl] = v;
-  }
+  for (; q < q1; ++q) s += P[(size_t)q * stride + o];
+  part[grp][lane] = s;
   __syncthreads();
-  // mirror: out(j, i) = value(i, j) for i < j; thread tx runs along j
+  double r = 0.0;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int il = ty + 8 * u, ii = 32 * bi + il, jj = 32 * bj + tx;
-    if (ii < n && jj < n && ii < jj) out[(size_t)ii * ldo + jj] = tile[il][tx];
-  }
+  for (int g = 0; g < 8; ++g) r += part[g][lane];
+  return r;
+}
+
+// out(i, j) = alpha sum_q P[q](i, j) [- A(0, i) B(0, j)], partials P[q] of ldp
+// rows (the first m used); symmetric (m == n, the upper triangle of P): also
+// out(j, i)
+__global__ __launch_bounds__(256) void k_reduce_tn(const double* __restrict__ P, int nsplit, int ldp, int m, int n,
+                                                   double alpha, const double* __restrict__ a0, int lda,
+                                                   const double* __restrict__ b0, int ldb, int g0, int symmetric,
+                                                   double* __restrict__ out, int ldo) {
+  const int i = blockIdx.x * 32 + (threadIdx.x & 31), j = blockIdx.y;
+  if (symmetric && (int)blockIdx.x * 32 > j) return;
+  const bool on = i < m && (!symmetric || i <= j);
+  const double s = sum_partials(P, nsplit, (size_t)ldp * n, (size_t)j * ldp + i, on);
+  if (!on || threadIdx.x >= 32) return;
+  double v = alpha * s;
+  if (g0) v -= a0[(size_t)i * lda] * b0[(size_t)j * ldb];
+  out[(size_t)j * ldo + i] = v;
+  if (symmetric && i != j) out[(size_t)i * ldo + j] = v;
+}
+
+// the projector contraction's partials to fnl(isa, iv, j) = 2 sum and
+// dfnl(isa, iv, k, j) = 2 tpiba sum (variant v0 + v = 0 and 1 + k)
+__global__ __launch_bounds__(256) void k_reduce_proj(const double* __restrict__ P, int nsplit, ProjTab t, int m, int n,
+                                                     int nat, int nhxs, double tpiba, double* __restrict__ fnl,
+                                                     double* __restrict__ dfnl) {
+  const int i = blockIdx.x * 32 + (threadIdx.x & 31), j = blockIdx.y;
+  const double s = sum_partials(P, nsplit, (size_t)m * n, (size_t)j * m + i, i < m);
+  if (i >= m || threadIdx.x >= 32) return;
+  const int v = t.v0 + i / t.ncol;
+  const int4 d = t.tab[i % t.ncol];
+  const int iv = d.w & 0xffff;
+  if (v == 0)
+    fnl[d.x + (size_t)nat * (iv + (size_t)nhxs * j)] = 2.0 * s;
+  else
+    dfnl[d.x + (size_t)nat * (iv + (size_t)nhxs * ((v - 1) + 3 * (size_t)j))] = 2.0 * tpiba * s;
 }
 
 // ---------------------------------------------------------------------------
@@ -372,10 +368,15 @@ void gemm_tn(mc_ctx* ctx, const double* A, int lda, const double* B, int ldb, in
     gemm_tn_x3(ctx, A, lda, B, ldb, K, m, n, alpha, g0corr, symmetric, out, ldo, proj);
     return;
   }
+  if (symmetric && m != n) throw Error{MC_ERR_INTERNAL, "symmetric A^T B with m != n"};
+  if (!proj && tn_f64_form(A, lda, B, ldb)) {
+    const int ns = tn_f64_partials(ctx, A, lda, B, ldb, K, m, n, symmetric, nullptr);
+    reduce_tn(ctx, ns, m, n, alpha, A, lda, B, ldb, g0corr, symmetric, out, ldo);
+    return;
+  }
   // 128-tiles for long K, 64-tiles (more workgroups) for short K
   const int BT = K >= 16384 ? 128 : 64;
   const int tm = (m + BT - 1) / BT, tn = (n + BT - 1) / BT;
-  if (symmetric && m != n) throw Error{MC_ERR_INTERNAL, "symmetric A^T B with m != n"};
   const int tiles = tile_count(symmetric, tm, tn);
   // about 1024 busy workgroups (4 per CU), K chunks of at least 512 rows
   int nsplit = std::max(1, std::min((1024 + tiles - 1) / tiles, std::max(1, K / 512)));
@@ -402,15 +403,7 @@ void gemm_tn(mc_ctx* ctx, const double* A, int lda, const double* B, int ldb, in
 void reduce_tn(mc_ctx* ctx, int nsplit, int m, int n, double alpha, const double* A, int lda, const double* B, int ldb,
                bool g0corr, bool symmetric, double* out, int ldo) {
   timer_begin(ctx, MC_KID_MISC);
-  if (symmetric && m == n) {
-    const int nb = (n + 31) / 32;
-    hipLaunchKernelGGL(k_reduce_tn_sym, dim3(nb * (nb + 1) / 2), dim3(256), 0, ctx->stream, ctx->w_gemm.as<double>(),
-                       nsplit, m, n, alpha, A, lda, B, ldb, g0corr ? 1 : 0, out, ldo);
-    MC_HIP(hipGetLastError());
-    timer_end(ctx, MC_KID_MISC);
-    return;
-  }
-  hipLaunchKernelGGL(k_reduce_tn, dim3((m + 255) / 256, n), dim3(256), 0, ctx->stream, ctx->w_gemm.as<double>(),
+  hipLaunchKernelGGL(k_reduce_tn, dim3((m + 31) / 32, n), dim3(256), 0, ctx->stream, ctx->w_gemm.as<double>(),
                      nsplit, m, m, n, alpha, A, lda, B, ldb, g0corr ? 1 : 0, symmetric ? 1 : 0, out, ldo);
   MC_HIP(hipGetLastError());
   timer_end(ctx, MC_KID_MISC);
@@ -418,8 +411,18 @@ void reduce_tn(mc_ctx* ctx, int nsplit, int m, int n, double alpha, const double
 
 void reduce_tn_rows(mc_ctx* ctx, int nsplit, int ldp, int r0, int m, int n, double alpha, double* out, int ldo) {
   timer_begin(ctx, MC_KID_MISC);
-  hipLaunchKernelGGL(k_reduce_tn, dim3((m + 255) / 256, n), dim3(256), 0, ctx->stream, ctx->w_gemm.as<double>() + r0,
+  hipLaunchKernelGGL(k_reduce_tn, dim3((m + 31) / 32, n), dim3(256), 0, ctx->stream, ctx->w_gemm.as<double>() + r0,
                      nsplit, ldp, m, n, alpha, (const double*)nullptr, 0, (const double*)nullptr, 0, 0, 0, out, ldo);
+  MC_HIP(hipGetLastError());
+  timer_end(ctx, MC_KID_MISC);
+}
+
+void reduce_proj(mc_ctx* ctx, int nsplit, const ProjTab& t, int nv, int n, int nat, int nhxs, double tpiba,
+                 double* fnl, double* dfnl) {
+  const int m = nv * t.ncol;
+  timer_begin(ctx, MC_KID_MISC);
+  hipLaunchKernelGGL(k_reduce_proj, dim3((m + 31) / 32, n), dim3(256), 0, ctx->stream, ctx->w_gemm.as<double>(),
+                     nsplit, t, m, n, nat, nhxs, tpiba, fnl, dfnl);
   MC_HIP(hipGetLastError());
   timer_end(ctx, MC_KID_MISC);
 }
@@ -447,6 +450,10 @@ void gemm_nn_f64(mc_ctx* ctx, const double* A, int lda, const double* G, int ldg
   if (M <= 0 || n <= 0) return;
   FnlEpi e{};
   if (epi) e = *epi;
+  if ((!e.twnl || beta != 0.0) && M >= 4096 && nn_f64_form(A, lda, M, D, ldd, &e)) {
+    nn_f64(ctx, A, lda, G, ldgm, M, k, n, alpha, beta, D, ldd, upper_g, e, nullptr, kid);
+    return;
+  }
   // 128-tiles when they already give >= 1024 workgroups, 64-tiles otherwise
   const int t128 = ((M + 127) / 128) * ((n + 127) / 128);
   const int BT = t128 >= 1024 ? 128 : 64;

@@ -159,6 +159,19 @@ struct ProjA {
   int n1 = 0, n2 = 0, n3 = 0, isa0 = 0;
 };
 
+// The projector operand of all (species, projector, atom) columns, built on
+// the fly by the FP64 contractions (gemm_f64.hip).  Column c of variant v =
+// c / ncol (v0 + v = 0: fnl and fnonloc, 1..3: dfnl along x, y, z) is
+// projector column c % ncol of tab: (atom, column of twnl, l mod 4, projector +
+// 2^16 times its species' number of projectors).
+struct ProjTab {
+  const int4* tab = nullptr;
+  const double2* eigr = nullptr;   // (ldg, nat)
+  const double* twnl = nullptr;    // (ldg, nhxs nsp)
+  const double* gk = nullptr;      // (ldg, 3)
+  int ncol = 1, v0 = 0, ldg = 0, geq0 = 0;
+};
+
 // Epilogue of fnonloc (src/fnonloc_utils.mod.F90:272-300):
 // c2(g,i) += twnl(g) ctm_i auxc(g,i), ctm_i = -f_i (-i)^l, f_i < 1e-5 -> 1.
 struct FnlEpi {
@@ -197,6 +210,10 @@ struct Projectors {
   DevBuf d_gk;     // (ldg, 3) G vectors in units of 2 pi / alat (rnlsm2)
   bool gk_ready = false;
   DevBuf d_dfnl;   // (nat, nhxs, 3, nstate)
+  // ProjTab::tab, ncol entries in (species, projector, atom) order, behind d_h's matrices
+  int ncol = 0;
+  size_t tab_off = 0;
+  const int4* tab() const { return reinterpret_cast<const int4*>(static_cast<const char*>(d_h.p) + tab_off); }
   int dfnl_nstate = -1;
 };
 
@@ -395,6 +412,16 @@ void reduce_tn(mc_ctx* ctx, int nsplit, int m, int n, double alpha, const double
                bool g0corr, bool symmetric, double* out, int ldo);
 // rows [r0, r0 + m) of partials with ldp rows: out = alpha sum of the nsplit partials
 void reduce_tn_rows(mc_ctx* ctx, int nsplit, int ldp, int r0, int m, int n, double alpha, double* out, int ldo);
+// FP64 products of aligned operands (gemm_f64.hip)
+bool tn_f64_form(const double* A, int lda, const double* B, int ldb);
+int tn_f64_partials(mc_ctx* ctx, const double* A, int lda, const double* B, int ldb, int K, int m, int n,
+                    bool symmetric, const ProjTab* proj);
+bool nn_f64_form(const double* A, int lda, int M, const double* D, int ldd, const FnlEpi* epi);
+void nn_f64(mc_ctx* ctx, const double* A, int lda, const double* G, int ldgm, int M, int k, int n, double alpha,
+            double beta, double* D, int ldd, bool upper_g, const FnlEpi& epi, const ProjTab* proj, int kid);
+// fnl (v0 = 0, first variant) and dfnl from the partials of the projector operand
+void reduce_proj(mc_ctx* ctx, int nsplit, const ProjTab& t, int nv, int n, int nat, int nhxs, double tpiba,
+                 double* fnl, double* dfnl);
 // split-bf16 (3-term, FP32 accumulation) variants used in mixed precision (gemm_x3.hip)
 constexpr int kX3Min = 16384;   // rows of K (tn) or M (nn) from which the split kernels are used
 // bf16 part planes and the contraction that streams them (gemm_planes.hip)

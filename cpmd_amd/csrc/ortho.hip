@@ -241,6 +241,23 @@ __global__ void k_fnl_dd(const double* __restrict__ fnl, int nat, int nhxs, int 
   dd[ia + (size_t)na * i] = s;
 }
 
+// dd(c, i) of every projector column c = (species, iv, ia) of tab
+__global__ void k_fnl_dd_all(const double* __restrict__ fnl, int nat, int nhxs, const int4* __restrict__ tab, int ncol,
+                             const double* __restrict__ h, double* __restrict__ dd) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y;
+  if (c >= ncol) return;
+  const int4 d = tab[c];
+  const int is = d.y / nhxs, iv = d.w & 0xffff, nh = d.w >> 16;
+  const double* hs = h + (size_t)nhxs * nhxs * is + iv;
+  const double* x = fnl + d.x + (size_t)nat * nhxs * i;
+  double s = 0.0;
+  for (int jv = 0; jv < nh; ++jv) {
+    const double hv = hs[nhxs * jv];
+    if (hv != 0.0) s += x[(size_t)nat * jv] * hv;
+  }
+  dd[c + (size_t)ncol * i] = s;
+}
+
 __global__ void k_permute_rows_in(const double2* __restrict__ src, int lds, double2* __restrict__ dst, int ldd,
                                   const int* __restrict__ perm, int ngw, int ncol) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y;
@@ -676,9 +693,23 @@ void set_projectors(mc_ctx* ctx, int nsp, const int* na, int nhxs, const int* ng
     P.nat += na[is];
   }
   const size_t nh = (size_t)nhxs * nhxs * nsp;
-  P.d_h.ensure(sizeof(double) * std::max<size_t>(nh, 1));
-  if (nh) MC_HIP(hipMemcpy(P.d_h.p, hmat, sizeof(double) * nh, hipMemcpyHostToDevice));
   P.h_h.assign(hmat, hmat + nh);
+  // one upload: hmat and, behind it, the projector columns in (species,
+  // projector, atom) order
+  MC_CHECK(nhxs < 0x8000, MC_ERR_ARG, "set_projectors: bad nhxs");
+  std::vector<int4> tab;
+  for (int is = 0, isa0 = 0; is < nsp; isa0 += na[is++])
+    for (int iv = 0; iv < ngh[is]; ++iv)
+      for (int ia = 0; ia < na[is]; ++ia)
+        tab.push_back(make_int4(isa0 + ia, is * nhxs + iv, ((lang[iv + (size_t)nhxs * is] % 4) + 4) % 4,
+                                iv | ngh[is] << 16));
+  P.ncol = (int)tab.size();
+  P.tab_off = (sizeof(double) * nh + 15) / 16 * 16;
+  std::vector<char> up(P.tab_off + sizeof(int4) * tab.size());
+  if (nh) std::copy_n((const char*)hmat, sizeof(double) * nh, up.data());
+  if (P.ncol) std::copy_n((const char*)tab.data(), sizeof(int4) * tab.size(), up.data() + P.tab_off);
+  P.d_h.ensure(std::max<size_t>(up.size(), 16));
+  if (!up.empty()) MC_HIP(hipMemcpy(P.d_h.p, up.data(), up.size(), hipMemcpyHostToDevice));
   // twnl (ngw, nhxs, nsp) in CPMD order -> device rows (ldg) in stick order
   const int ncol = nhxs * nsp;
   P.d_twnl.ensure(sizeof(double) * (size_t)ctx->ldg * std::max(ncol, 1));
@@ -711,12 +742,29 @@ void set_eigr(mc_ctx* ctx, const double* eigr, int lde, int nat) {
   MC_HIP(hipStreamSynchronize(ctx->stream));
 }
 
+static ProjTab proj_tab(const mc_ctx* ctx, int v0) {
+  const auto& P = ctx->proj;
+  ProjTab t;
+  t.tab = P.tab();
+  t.eigr = P.d_eigr.as<double2>();
+  t.twnl = P.d_twnl.as<double>();
+  t.gk = P.d_gk.as<double>();
+  t.ncol = std::max(P.ncol, 1);
+  t.v0 = v0;
+  t.ldg = ctx->ldg;
+  t.geq0 = ctx->geq0;
+  return t;
+}
+
 // fnl(isa, iv, i) = 2 Re sum_G conj((-i)^l twnl eigr) c (rnlsm1,
 // src/rnlsm1_utils.mod.F90:42-193) and dfnl(isa, iv, k, i) = 2 tpiba Re sum_G
 // conj(gk_k twnl (-i)^(l+1) eigr) c (rnlsm2, src/rnlsm2_utils.mod.F90:321-482),
 // G = 0 halved, per (species, projector) group.  In mixed precision the
 // requested variants of a group are one stacked split-bf16 contraction over
-// the planes of c0.
+// the planes of c0; in FP64 every group and variant is one contraction (64
+// atoms of two species with s and p projectors, 130 states at 128^3, fnl and
+// dfnl: 0.68 ms where a product per group and variant took 6.3 ms, most of it
+// on the padding of 21 and 43 columns to 128).
 static void rnlsm_groups(mc_ctx* ctx, const double2* c0, int n, bool do_fnl, bool do_dfnl, double* fnl_host,
                          double* dfnl_host) {
   auto& P = ctx->proj;
@@ -725,16 +773,20 @@ static void rnlsm_groups(mc_ctx* ctx, const double2* c0, int n, bool do_fnl, boo
   MC_CHECK(P.eigr_nat == P.nat, MC_ERR_ARG, "rnlsm: structure factors not set for all atoms (mc_set_eigr)");
   MC_CHECK(!do_dfnl || P.gk_ready, MC_ERR_ARG, "rnlsm2: G vectors not set (mc_set_gk)");
   const size_t nf = (size_t)P.nat * P.nhxs * std::max(n, 1);
+  // entries no projector writes (ngh < nhxs of some species) stay zero
+  const bool full = n > 0 && P.ncol == P.nat * P.nhxs;
   if (do_fnl) {
     P.d_fnl.ensure(sizeof(double) * nf);
     P.fnl_nstate = n;
-    hipLaunchKernelGGL(k_zero, dim3(64), dim3(256), 0, ctx->stream, P.d_fnl.as<double>(), nf);
+    if (!full)
+      hipLaunchKernelGGL(k_zero, dim3(64), dim3(256), 0, ctx->stream, P.d_fnl.as<double>(), nf);
     MC_HIP(hipGetLastError());
   }
   if (do_dfnl) {
     P.d_dfnl.ensure(sizeof(double) * nf * 3);
     P.dfnl_nstate = n;
-    hipLaunchKernelGGL(k_zero, dim3(64), dim3(256), 0, ctx->stream, P.d_dfnl.as<double>(), nf * 3);
+    if (!full)
+      hipLaunchKernelGGL(k_zero, dim3(64), dim3(256), 0, ctx->stream, P.d_dfnl.as<double>(), nf * 3);
     MC_HIP(hipGetLastError());
   }
   const double tpiba = std::sqrt(ctx->tpiba2);
@@ -742,8 +794,15 @@ static void rnlsm_groups(mc_ctx* ctx, const double2* c0, int n, bool do_fnl, boo
   const double* B = (const double*)c0;
   const bool x3 = ctx->gemm_x3 && K >= kX3Min;
   const int ldf = P.nat * P.nhxs, ldd = P.nat * P.nhxs * 3;
+  const bool stacked = !x3 && tn_f64_form(B, ldb, B, ldb);
+  if (stacked && P.ncol > 0 && n > 0) {
+    const ProjTab t = proj_tab(ctx, do_fnl ? 0 : 1);
+    const int nv = (do_fnl ? 1 : 0) + (do_dfnl ? 3 : 0);
+    const int ns = tn_f64_partials(ctx, nullptr, 0, B, ldb, K, nv * P.ncol, n, false, &t);
+    reduce_proj(ctx, ns, t, nv, n, P.nat, P.nhxs, tpiba, P.d_fnl.as<double>(), P.d_dfnl.as<double>());
+  }
   int isa0 = 0;
-  for (int is = 0; is < P.nsp; ++is) {
+  for (int is = 0; is < P.nsp && !stacked; ++is) {
     for (int iv = 0; iv < P.ngh[is]; ++iv) {
       if (P.na[is] == 0 || n == 0) continue;
       ProjA pa;
@@ -908,6 +967,28 @@ void fnonloc_dev(mc_ctx* ctx, double2* c2, const double* f_host, int n, const do
   MC_CHECK(P.fnl_nstate == n, MC_ERR_ARG, "fnonloc: no fnl for this number of states (call rnlsm1 first)");
   ctx->w_f2.ensure(sizeof(double) * n);
   MC_HIP(hipMemcpyAsync(ctx->w_f2.p, f_host, sizeof(double) * n, hipMemcpyHostToDevice, ctx->stream));
+  const int M = wfn_rows(ctx);
+  int groups = 0;
+  for (int is = 0; is < P.nsp; ++is) groups += P.na[is] > 0 ? P.ngh[is] : 0;
+  if (groups > 1 && !(ctx->gemm_x3 && M >= kX3Min) && nn_f64_form((const double*)c2, wfn_ld(ctx), M, (const double*)c2, wfn_ld(ctx), nullptr)) {
+    // one product over all projector columns: c2 is read and written once (64
+    // atoms of two species, 5 projectors, 130 states at 128^3: 0.27 ms against
+    // 1.26 ms for a product per projector).  A single group takes the plain
+    // product below, its factor applied to the result: eigr is then copied to
+    // LDS as it is (256 atoms, 512 states, 192^3: 2.06 against 2.58 ms)
+    if (P.ncol == 0) return;
+    ctx->w_dd.ensure(sizeof(double) * (size_t)P.ncol * n);
+    hipLaunchKernelGGL(k_fnl_dd_all, dim3((P.ncol + 63) / 64, n), dim3(64), 0, ctx->stream, P.d_fnl.as<double>(),
+                       P.nat, P.nhxs, P.tab(), P.ncol, P.d_h.as<double>(),
+                       ctx->w_dd.as<double>());
+    MC_HIP(hipGetLastError());
+    const ProjTab t = proj_tab(ctx, 0);
+    FnlEpi e{};
+    e.f = ctx->w_f2.as<double>();
+    nn_f64(ctx, nullptr, 0, ctx->w_dd.as<double>(), P.ncol, M, P.ncol, n, 1.0, 1.0, (double*)c2, wfn_ld(ctx), false, e,
+           &t, MC_KID_GEMM);
+    return;
+  }
   int namax = 0;
   for (int is = 0; is < P.nsp; ++is) namax = std::max(namax, P.na[is]);
   ctx->w_dd.ensure(sizeof(double) * (size_t)std::max(namax, 1) * n);
