@@ -7,6 +7,8 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -14,7 +16,8 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libmicpmd.so"
 
-HIP_SOURCES = ["context.hip", "wfft.hip", "gemm.hip", "gemm_f64.hip", "gemm_x3.hip", "gemm_planes.hip", "ortho.hip", "vofrho.hip",
+HIP_SOURCES = ["context.hip", "wfft.hip", *(f"wfft_len_{i}.hip" for i in range(1, 8)), "gemm.hip",
+               "gemm_f64.hip", "gemm_x3.hip", "gemm_planes.hip", "ortho.hip", "vofrho.hip",
                "capi.hip", "restart.hip", "probe.hip"]
 
 HIPCC_FLAGS = [
@@ -22,7 +25,6 @@ HIPCC_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     # packed FP32 instructions are kept out of every kernel
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-result", "-Wno-unused-function",
@@ -68,10 +70,7 @@ def build_fortran(verbose: bool = False) -> Path:
     return DRIVER
 
 
-def build(verbose: bool = False) -> Path:
-    srcs = [str(CSRC / s) for s in HIP_SOURCES]
-    tmp = LIB.with_suffix(".so.tmp")
-    cmd = [hipcc(), *HIPCC_FLAGS, "-I", str(ROOT / "include"), *srcs, "-o", str(tmp)]
+def run(cmd: list, verbose: bool):
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -83,6 +82,22 @@ def build(verbose: bool = False) -> Path:
         lines = [l for l in (r.stdout + r.stderr).splitlines() if "packed-fp32-ops" not in l]
         if lines:
             print("\n".join(lines))
+
+
+def build(verbose: bool = False) -> Path:
+    tmp = LIB.with_suffix(".so.tmp")
+    with tempfile.TemporaryDirectory() as d:
+        # one object per source, several at a time (the transform lengths
+        # dominate: one process takes minutes for all)
+        objs = [Path(d) / (Path(s).stem + ".o") for s in HIP_SOURCES]
+
+        def compile_one(src, obj):
+            return run([hipcc(), *HIPCC_FLAGS, "-I", str(ROOT / "include"), "-c", str(CSRC / src), "-o", str(obj)],
+                       verbose)
+
+        with ThreadPoolExecutor(max(1, min(8, os.cpu_count() or 1))) as pool:
+            list(pool.map(compile_one, HIP_SOURCES, objs))
+        run([hipcc(), "--offload-arch=gfx950", "-fPIC", "-shared", *map(str, objs), "-o", str(tmp)], verbose)
     os.replace(tmp, LIB)
     return LIB
 

@@ -8,7 +8,7 @@
 //
 // Two engines, both cooperative over one workgroup of kThreads threads on a
 // batch of lines held in LDS (line stride `lds`):
-//  * fft_fast<T, N, DIR>: lengths N = A*B known at compile time (A, B <= 16).
+//  * fft_fast<T, N, DIR>: lengths N = A*B known at compile time (A, B <= 20).
 //    Four-step: each thread does one length-A DFT in registers over x[B n1 + n2]
 //    (stride B), multiplies by w_N^{n2 k1}, the lines are transposed in LDS and
 //    each thread does one length-B DFT in registers.  Two LDS round trips per
@@ -237,6 +237,32 @@ __device__ __forceinline__ void dft16_band(V* v) {
   }
 }
 
+// As dft16_band<DIR, true, false> for any A = 4 Q: the inputs Q .. 3Q - 1 are
+// zero and not read.
+template <int A, int DIR, typename V>
+__device__ __forceinline__ void dft_band_in(V* v) {
+  constexpr int Q = A / 4;
+  static_assert(A % 4 == 0 && A > 4, "band DFT of a length 4 Q");
+  V y[A];
+#pragma unroll
+  for (int n2 = 0; n2 < Q; ++n2) {
+    const V a = v[n2], d = v[3 * Q + n2];
+    const V md = mul_di<DIR>(d);
+    const V u[4] = {cadd(a, d), csub(a, md), csub(a, d), cadd(a, md)};
+#pragma unroll
+    for (int k1 = 0; k1 < 4; ++k1) y[n2 * 4 + k1] = ((n2 * k1) % A == 0) ? u[k1] : twc<A, DIR>(u[k1], (n2 * k1) % A);
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < 4; ++k1) {
+    V u[Q];
+#pragma unroll
+    for (int n2 = 0; n2 < Q; ++n2) u[n2] = y[n2 * 4 + k1];
+    dftn<Q, DIR>(u);
+#pragma unroll
+    for (int k2 = 0; k2 < Q; ++k2) v[k1 + 4 * k2] = u[k2];
+  }
+}
+
 // ---------------------------------------------------------------------------
 // compile-time four-step engine
 // ---------------------------------------------------------------------------
@@ -251,9 +277,44 @@ MC_FAST_SHAPE(128, 16, 8)
 MC_FAST_SHAPE(192, 16, 12)
 MC_FAST_SHAPE(224, 16, 14)
 MC_FAST_SHAPE(240, 16, 15)
+MC_FAST_SHAPE(30, 6, 5)
+MC_FAST_SHAPE(32, 8, 4)
+MC_FAST_SHAPE(36, 6, 6)
+MC_FAST_SHAPE(40, 8, 5)
+MC_FAST_SHAPE(48, 8, 6)
+MC_FAST_SHAPE(60, 10, 6)
+MC_FAST_SHAPE(64, 8, 8)
+MC_FAST_SHAPE(72, 8, 9)
+MC_FAST_SHAPE(80, 8, 10)
+MC_FAST_SHAPE(90, 10, 9)
+MC_FAST_SHAPE(96, 12, 8)
+MC_FAST_SHAPE(100, 10, 10)
+MC_FAST_SHAPE(108, 12, 9)
+MC_FAST_SHAPE(120, 12, 10)
+MC_FAST_SHAPE(144, 12, 12)
+MC_FAST_SHAPE(150, 15, 10)
+MC_FAST_SHAPE(160, 16, 10)
+MC_FAST_SHAPE(162, 18, 9)
+MC_FAST_SHAPE(180, 12, 15)
+MC_FAST_SHAPE(200, 20, 10)
+MC_FAST_SHAPE(216, 12, 18)
+MC_FAST_SHAPE(256, 16, 16)
+MC_FAST_SHAPE(270, 18, 15)
+MC_FAST_SHAPE(288, 16, 18)
+MC_FAST_SHAPE(300, 20, 15)
+MC_FAST_SHAPE(320, 16, 20)
 #undef MC_FAST_SHAPE
-// the lengths with a compile-time engine (host dispatch lists the same)
+// The lengths with a compile-time engine: both arithmetic types, and FP64
+// only.  The second list is the rest of CPMD's even default lengths from 30 to
+// 320, i.e. the meshes of cells of any edge, with factors A = 4 Q where the two
+// stay close (band pruning).  Density of 103 states on 108 x 120 x 160: 0.65 ms
+// against 3.69 ms with the runtime-plan engine, whose stages divide by runtime
+// lengths for every butterfly and pass through LDS three to five times.  FP32
+// keeps the runtime plan at these lengths: its rounding differs.
 #define MC_FAST_SIZES(X) X(16) X(18) X(24) X(54) X(128) X(192) X(224) X(240)
+#define MC_F64_SIZES(X)                                                                                    \
+  X(30) X(32) X(36) X(40) X(48) X(60) X(64) X(72) X(80) X(90) X(96) X(100) X(108) X(120) X(144) X(150) X(160) \
+  X(162) X(180) X(200) X(216) X(256) X(270) X(288) X(300) X(320)
 
 // In-place transform of `nlines` lines (line stride lds) with tw = LDS copy of
 // the N-point table; nlines * A <= kThreads.  Begins and ends with a barrier
@@ -368,14 +429,22 @@ inline int max_lines(const FftPlan& pl) {
   return (kMaxBfly * kThreads * rmin) / pl.n;
 }
 
-// Host side: the fast-engine factor A of length n (0 when n has no compile-time engine).
+// Host side: lanes per line of the fast engine of length n (its larger
+// factor; 0 when n has no compile-time engine for arithmetic type T).
+template <typename T>
 inline int fast_a(int n) {
+#define MC_CASE(x) case x: return FastShape<x>::A > FastShape<x>::B ? FastShape<x>::A : FastShape<x>::B;
+  if (sizeof(T) == 8) {
+    switch (n) {
+      MC_F64_SIZES(MC_CASE)
+      default: break;
+    }
+  }
   switch (n) {
-#define MC_CASE(x) case x: return FastShape<x>::A;
     MC_FAST_SIZES(MC_CASE)
-#undef MC_CASE
     default: return 0;
   }
+#undef MC_CASE
 }
 
 }  // namespace mc

@@ -39,7 +39,7 @@ constexpr int kLdsBudget = 65536;
 // lines per workgroup for a transform of length n: engine limits, LDS (lines + table) and 16
 template <typename T>
 inline int lines_for(const FftPlan& pl) {
-  const int a = fast_a(pl.n);
+  const int a = fast_a<T>(pl.n);
   int l = a > 0 ? kThreads / a : max_lines(pl);
   l = std::min(l, kLdsBudget / (int)(sizeof(v2<T>) * pl.n) - 1);
   l = std::min(l, 16);
@@ -49,16 +49,22 @@ inline int lines_for(const FftPlan& pl) {
 
 
 // calls f(std::integral_constant<int, N>) with N = n if n has a compile-time
-// engine, N = 0 otherwise
-template <class F>
+// engine for arithmetic type T, N = 0 otherwise
+template <typename T, class F>
 inline void with_length(int n, F&& f) {
-  switch (n) {
 #define MC_CASE(x) \
   case x: f(std::integral_constant<int, x>()); return;
+  if constexpr (sizeof(T) == 8) {
+    switch (n) {
+      MC_F64_SIZES(MC_CASE)
+      default: break;
+    }
+  }
+  switch (n) {
     MC_FAST_SIZES(MC_CASE)
-#undef MC_CASE
     default: f(std::integral_constant<int, 0>()); return;
   }
+#undef MC_CASE
 }
 
 #define LAUNCH(kid, kern, grid, block, shm, ...)                                  \

@@ -4,7 +4,7 @@ Run: python cpmd_amd/csrc/gen_twiddles.py > cpmd_amd/csrc/twiddle_consts.h"""
 from decimal import Decimal, getcontext
 
 getcontext().prec = 60
-SIZES = (6, 7, 8, 9, 10, 12, 14, 15, 16, 21, 28)
+SIZES = (6, 7, 8, 9, 10, 12, 14, 15, 16, 18, 20, 21, 28)
 
 
 def pi():

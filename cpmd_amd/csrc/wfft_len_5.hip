@@ -1,0 +1,13 @@
+// Transform passes of the lengths below (compile-time engines; see wfft_passes.h)
+#include "wfft_passes.h"
+
+namespace mc {
+
+template struct Passes<double, 100>;
+template struct Passes<double, 108>;
+template struct Passes<double, 120>;
+template struct Passes<double, 144>;
+template struct Passes<double, 150>;
+template struct Passes<double, 160>;
+
+}  // namespace mc

@@ -1,0 +1,12 @@
+// Transform passes of the lengths below (compile-time engines; see wfft_passes.h)
+#include "wfft_passes.h"
+
+namespace mc {
+
+template struct Passes<double, 162>;
+template struct Passes<double, 180>;
+template struct Passes<double, 200>;
+template struct Passes<double, 216>;
+template struct Passes<double, 256>;
+
+}  // namespace mc
