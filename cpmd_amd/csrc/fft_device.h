@@ -6,14 +6,16 @@
 // (r -> G) is e^{-i 2 pi k x / n}; the 1/(n1 n2 n3) scale is applied by the
 // caller after the last forward pass.
 //
-// Two engines, both cooperative over one workgroup of kThreads threads on a
+// Three engines, all cooperative over one workgroup of kThreads threads on a
 // batch of lines held in LDS (line stride `lds`):
-//  * fft_fast<T, N, DIR>: lengths N = A*B known at compile time (A, B <= 20).
-//    Four-step: each thread does one length-A DFT in registers over x[B n1 + n2]
-//    (stride B), multiplies by w_N^{n2 k1}, the lines are transposed in LDS and
-//    each thread does one length-B DFT in registers.  Two LDS round trips per
-//    transform.  Register DFTs of composite length recurse at compile time into
-//    radix 2/3/4/5/7 butterflies with exact constant twiddles (twiddle_consts.h).
+//  * fft_fast<T, N, DIR>: lengths N = A*B known at compile time, two LDS round
+//    trips per transform.  Four-step form (A, B <= 20): each thread does one
+//    length-A DFT in registers over x[B n1 + n2] (stride B), multiplies by
+//    w_N^{n2 k1}, the lines are transposed in LDS and each thread does one
+//    length-B DFT in registers.  Register DFTs of composite length recurse at
+//    compile time into radix 2/3/4/5/7 butterflies with exact constant twiddles
+//    (twiddle_consts.h).  Stage form (FP32 at the lengths of MC_MORE_SIZES): the
+//    stages of the runtime plan, grouped A and B points at a time in registers.
 //  * fft_lines<T, DIR>: any 2^a 3^b 5^c 7^d length from a runtime plan: mixed-radix
 //    Stockham stages; stage s with radix R and p = product of previous radices
 //    maps butterfly i of a line to inputs x[i + q n/R], twiddles w^{q k n/(pR)}
@@ -304,25 +306,143 @@ MC_FAST_SHAPE(288, 16, 18)
 MC_FAST_SHAPE(300, 20, 15)
 MC_FAST_SHAPE(320, 16, 20)
 #undef MC_FAST_SHAPE
-// The lengths with a compile-time engine: both arithmetic types, and FP64
-// only.  The second list is the rest of CPMD's even default lengths from 30 to
-// 320, i.e. the meshes of cells of any edge, with factors A = 4 Q where the two
-// stay close (band pruning).  Density of 103 states on 108 x 120 x 160: 0.65 ms
-// against 3.69 ms with the runtime-plan engine, whose stages divide by runtime
-// lengths for every butterfly and pass through LDS three to five times.  FP32
-// keeps the runtime plan at these lengths: its rounding differs.
+// The lengths with a compile-time engine.  The second list is the rest of
+// CPMD's even default lengths from 30 to 320, i.e. the meshes of cells of any
+// edge, with factors A = 4 Q where the two stay close (band pruning).  The
+// runtime-plan engine divides by runtime lengths for every butterfly and passes
+// through LDS three to five times: density of 103 states on 108 x 120 x 160 in
+// FP64 0.65 against 3.69 ms, gradient of 61 states on 80 x 144 x 96 with FP32
+// transforms 0.33 against 1.08 ms.
 #define MC_FAST_SIZES(X) X(16) X(18) X(24) X(54) X(128) X(192) X(224) X(240)
-#define MC_F64_SIZES(X)                                                                                    \
+#define MC_MORE_SIZES(X)                                                                                    \
   X(30) X(32) X(36) X(40) X(48) X(60) X(64) X(72) X(80) X(90) X(96) X(100) X(108) X(120) X(144) X(150) X(160) \
   X(162) X(180) X(200) X(216) X(256) X(270) X(288) X(300) X(320)
 
+// The radices of the runtime plan (make_plan) of length N, and the split A B of
+// its stages that stays closest: A the product of the first stages, radix 5 left
+// to the second group (100 = 20 x 5 does not round as the plan's kernels do, 4 x
+// 25 does)
+struct StageList {
+  int nf = 0;
+  int rad[kMaxStages] = {};
+};
+constexpr StageList stage_list(int n) {
+  StageList s;
+  for (int r : {4, 2, 3, 5, 7})
+    while (n % r == 0) {
+      s.rad[s.nf++] = r;
+      n /= r;
+    }
+  return s;
+}
+constexpr int stage_split(int n) {
+  const StageList s = stage_list(n);
+  int best = 1, p = 1;
+  for (int i = 0; i < s.nf; ++i) {
+    p *= s.rad[i];
+    if (s.rad[i] == 5) break;
+    const int cur = best > n / best ? best : n / best, now = p > n / p ? p : n / p;
+    if (now <= cur) best = p;
+  }
+  return best;
+}
+
+// Which compile-time engine length N has: the four-step one (FP64, and FP32 at
+// the lengths of MC_FAST_SIZES) or, in FP32 at the others, the stages of the
+// runtime plan two groups at a time in registers (StockShape): the same
+// operations on the same values, so the results are those of the runtime plan
+// bit for bit.
+template <typename T, int N>
+constexpr bool four_step() {
+  if (sizeof(T) == 8) return true;
+#define MC_CASE(x) if (N == x) return true;
+  MC_FAST_SIZES(MC_CASE)
+#undef MC_CASE
+  return false;
+}
+template <typename T, int N>
+struct Shape {
+  static constexpr int A = four_step<T, N>() ? FastShape<N>::A : stage_split(N);
+  static constexpr int B = N / A;
+};
+
+// Keeps the compiler from merging arithmetic across this point (no
+// instruction): the runtime plan stores to LDS between its stages, and a product
+// or sum combined or vectorised across a stage boundary rounds differently.
+__device__ __forceinline__ void stage_end(float2& v) { asm("" : "+v"(v.x), "+v"(v.y)); }
+
+// twmul with the products that the compiler fuses in the runtime plan's kernels
+// written out: left to it, vectorised code fuses the other ones
+template <int DIR>
+__device__ __forceinline__ float2 twmul_stage(float2 a, float2 w) {
+  if (DIR < 0)
+    return make_float2(__builtin_fmaf(a.x, w.x, -(a.y * w.y)), __builtin_fmaf(a.y, w.x, a.x * w.y));
+  return make_float2(__builtin_fmaf(a.x, w.x, a.y * w.y), __builtin_fmaf(a.y, w.x, -(a.x * w.y)));
+}
+
+// Stages [S0, S0 + ...) of the runtime plan on the A (or B) values one thread
+// holds: v of length LEN, local product P of the stages done here, p = P * K
+// overall with this thread's k = k0 + K (0 .. P-1); tw: the N-point table.
+// IN (first stage a radix 4): the values LEN/4 .. 3 LEN/4 - 1 are zero and not read.
+template <int N, int S, int LEN, int P, int K, int DIR, bool IN, typename V>
+__device__ __forceinline__ void stock_stages(V* v, int k0, const V* tw) {
+  if constexpr (P < LEN) {
+    constexpr int R = stage_list(N).rad[S];
+    constexpr int M = LEN / (P * R);
+    static_assert(LEN % (P * R) == 0, "stages of the group");
+    V y[LEN];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int kk = 0; kk < P; ++kk) {
+        V u[R];
+        if constexpr (IN && P == 1) {
+          static_assert(R == 4, "band of a radix-4 first stage");
+          const V a = v[m], d = v[m + 3 * M];
+          const V md = mul_di<DIR>(d);
+          u[0] = cadd(a, d);
+          u[1] = csub(a, md);
+          u[2] = csub(a, d);
+          u[3] = cadd(a, md);
+        } else {
+#pragma unroll
+          for (int q = 0; q < R; ++q) u[q] = v[(m + q * M) * P + kk];
+          if constexpr (P * K > 1) {
+            const int k = k0 + K * kk;
+            if (K > 1 || kk > 0) {
+#pragma unroll
+              for (int q = 1; q < R; ++q) u[q] = twmul_stage<DIR>(u[q], tw[q * k * (N / (P * K * R))]);
+            }
+          }
+          dftn<R, DIR>(u);
+        }
+#pragma unroll
+        for (int q = 0; q < R; ++q) y[m * P * R + kk + q * P] = u[q];
+      }
+#pragma unroll
+    for (int i = 0; i < LEN; ++i) {
+      v[i] = y[i];
+      stage_end(v[i]);
+    }
+    stock_stages<N, S + 1, LEN, P * R, K, DIR, IN, V>(v, k0, tw);
+  }
+}
+// index of the first stage of the second group
+template <int N, int A>
+constexpr int second_stage() {
+  const StageList s = stage_list(N);
+  int p = 1, i = 0;
+  while (p < A) p *= s.rad[i++];
+  return i;
+}
+
 // In-place transform of `nlines` lines (line stride lds) with tw = LDS copy of
-// the N-point table; nlines * A <= kThreads.  Begins and ends with a barrier
+// the N-point table; nlines * max(A, B) <= kThreads.  Begins and ends with a barrier
 // point (callers synchronise before, this returns after a __syncthreads).
 template <typename T, int N, int DIR>
 __device__ __forceinline__ void fft_fast(v2<T>* buf, int nlines, int lds, const v2<T>* tw) {
   using V = v2<T>;
-  constexpr int A = FastShape<N>::A, B = FastShape<N>::B;
+  constexpr int A = Shape<T, N>::A, B = Shape<T, N>::B;
   static_assert(A * B == N && A >= 1 && B >= 1, "unsupported fast length");
   V v[A];
   const int t = threadIdx.x;
@@ -333,9 +453,13 @@ __device__ __forceinline__ void fft_fast(v2<T>* buf, int nlines, int lds, const 
   if (act1) {
 #pragma unroll
     for (int n1 = 0; n1 < A; ++n1) v[n1] = x1[B * n1 + n2];
-    dftn<A, DIR>(v);
+    if constexpr (four_step<T, N>()) {
+      dftn<A, DIR>(v);
 #pragma unroll
-    for (int k1 = 1; k1 < A; ++k1) v[k1] = twmul<DIR>(v[k1], tw[n2 * k1]);
+      for (int k1 = 1; k1 < A; ++k1) v[k1] = twmul<DIR>(v[k1], tw[n2 * k1]);
+    } else {
+      stock_stages<N, 0, A, 1, 1, DIR, false>(v, 0, tw);
+    }
   }
   __syncthreads();
   if (act1) {
@@ -351,7 +475,8 @@ __device__ __forceinline__ void fft_fast(v2<T>* buf, int nlines, int lds, const 
   if (act2) {
 #pragma unroll
     for (int m = 0; m < B; ++m) u[m] = x2[k1 * B + m];
-    dftn<B, DIR>(u);
+    if constexpr (four_step<T, N>()) dftn<B, DIR>(u);
+    else stock_stages<N, second_stage<N, A>(), B, 1, A, DIR, false>(u, k1, tw);
   }
   __syncthreads();
   if (act2) {
@@ -429,19 +554,14 @@ inline int max_lines(const FftPlan& pl) {
   return (kMaxBfly * kThreads * rmin) / pl.n;
 }
 
-// Host side: lanes per line of the fast engine of length n (its larger
-// factor; 0 when n has no compile-time engine for arithmetic type T).
+// Host side: lanes per line of the compile-time engine of length n (its larger
+// factor; 0 when n has none).
 template <typename T>
 inline int fast_a(int n) {
-#define MC_CASE(x) case x: return FastShape<x>::A > FastShape<x>::B ? FastShape<x>::A : FastShape<x>::B;
-  if (sizeof(T) == 8) {
-    switch (n) {
-      MC_F64_SIZES(MC_CASE)
-      default: break;
-    }
-  }
+#define MC_CASE(x) case x: return Shape<T, x>::A > Shape<T, x>::B ? Shape<T, x>::A : Shape<T, x>::B;
   switch (n) {
     MC_FAST_SIZES(MC_CASE)
+    MC_MORE_SIZES(MC_CASE)
     default: return 0;
   }
 #undef MC_CASE

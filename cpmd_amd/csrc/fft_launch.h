@@ -49,19 +49,14 @@ inline int lines_for(const FftPlan& pl) {
 
 
 // calls f(std::integral_constant<int, N>) with N = n if n has a compile-time
-// engine for arithmetic type T, N = 0 otherwise
-template <typename T, class F>
+// engine, N = 0 otherwise
+template <class F>
 inline void with_length(int n, F&& f) {
 #define MC_CASE(x) \
   case x: f(std::integral_constant<int, x>()); return;
-  if constexpr (sizeof(T) == 8) {
-    switch (n) {
-      MC_F64_SIZES(MC_CASE)
-      default: break;
-    }
-  }
   switch (n) {
     MC_FAST_SIZES(MC_CASE)
+    MC_MORE_SIZES(MC_CASE)
     default: f(std::integral_constant<int, 0>()); return;
   }
 #undef MC_CASE

@@ -693,15 +693,15 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
   gs.sf = Sf;
 
   // forward transform of rho
-  with_length<double>(ctx->n1, [&](auto NN) {
+  with_length(ctx->n1, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dx_fwd_real<decltype(NN)::value>), dim3(gx_blocks, ctx->n3), dim3(kThreads), shx, d,
            rho, W, tx);
   });
-  with_length<double>(ctx->n2, [&](auto NN) {
+  with_length(ctx->n2, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dyz<decltype(NN)::value, -1, 2>), dim3((ctx->n1 + t2 - 1) / t2, ctx->n3),
            dim3(kThreads), sh2, d, W, t2);
   });
-  with_length<double>(ctx->n3, [&](auto NN) {
+  with_length(ctx->n3, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dyz<decltype(NN)::value, -1, 3>), dim3((ctx->n1 + t3 - 1) / t3, ctx->n2),
            dim3(kThreads), sh3, d, W, t3);
   });
@@ -730,15 +730,15 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
   }
   LAUNCH(MC_KID_VOFRHO, k_fill, dim3(1024), dim3(256), 0, (double*)W, 2 * nw, 0.0);
   LAUNCH(MC_KID_VOFRHO, k_scatter_vtemp, dim3(kRedBlocks), dim3(kThreads), 0, g, vtemp, W);
-  with_length<double>(ctx->n3, [&](auto NN) {
+  with_length(ctx->n3, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dyz<decltype(NN)::value, 1, 3>), dim3((ctx->n1 + t3 - 1) / t3, ctx->n2),
            dim3(kThreads), sh3, d, W, t3);
   });
-  with_length<double>(ctx->n2, [&](auto NN) {
+  with_length(ctx->n2, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dyz<decltype(NN)::value, 1, 2>), dim3((ctx->n1 + t2 - 1) / t2, ctx->n3),
            dim3(kThreads), sh2, d, W, t2);
   });
-  with_length<double>(ctx->n1, [&](auto NN) {
+  with_length(ctx->n1, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dx_inv_xc<decltype(NN)::value>), dim3(gx_blocks, ctx->n3), dim3(kThreads), shx, d,
            W, rho, v, tx, p_xc);
   });

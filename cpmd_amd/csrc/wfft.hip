@@ -199,11 +199,11 @@ static void rhoofr_impl(mc_ctx* ctx, const double2* c0, const double* f_host, in
   for (int pair0 = 0; pair0 < npairs; pair0 += P) {
     const int np = std::min(P, npairs - pair0);
     V* B = K ? K + (size_t)pair0 * bslab : ctx->w_b.as<V>();
-    with_length<T>(ctx->n3, [&](auto NN) {
+    with_length(ctx->n3, [&](auto NN) {
       Passes<T, decltype(NN)::value>::zinv(ctx, w, s, np, c0, nstate, pair0, A, red + (size_t)pair0 * s.gx * 4);
     });
-    with_length<T>(ctx->n2, [&](auto NN) { Passes<T, decltype(NN)::value>::yinv(ctx, w, s, A, B, np); });
-    with_length<T>(ctx->n1, [&](auto NN) {
+    with_length(ctx->n2, [&](auto NN) { Passes<T, decltype(NN)::value>::yinv(ctx, w, s, A, B, np); });
+    with_length(ctx->n1, [&](auto NN) {
       Passes<T, decltype(NN)::value>::xrho(ctx, w, s, B, np, pair0, nstate, ctx->w_f.as<double>(), rho);
     });
   }
@@ -262,14 +262,14 @@ static void vpsi_run(mc_ctx* ctx, const double2* c0, double2* c2, const double* 
     if (K) {   // the inverse z and y passes of rhoofr, kept: start from its columns
       B = K + (size_t)pair0 * bslab;
     } else {
-      with_length<T>(ctx->n3, [&](auto NN) {
+      with_length(ctx->n3, [&](auto NN) {
         Passes<T, decltype(NN)::value>::zinv(ctx, w, s, np, c0, nstate, pair0, A, nullptr);
       });
-      with_length<T>(ctx->n2, [&](auto NN) { Passes<T, decltype(NN)::value>::yinv(ctx, w, s, A, B, np); });
+      with_length(ctx->n2, [&](auto NN) { Passes<T, decltype(NN)::value>::yinv(ctx, w, s, A, B, np); });
     }
-    with_length<T>(ctx->n1, [&](auto NN) { Passes<T, decltype(NN)::value>::xvpsi(ctx, w, s, B, np, vpot); });
-    with_length<T>(ctx->n2, [&](auto NN) { Passes<T, decltype(NN)::value>::yfwd(ctx, w, s, A, B, np); });
-    with_length<T>(ctx->n3, [&](auto NN) {
+    with_length(ctx->n1, [&](auto NN) { Passes<T, decltype(NN)::value>::xvpsi(ctx, w, s, B, np, vpot); });
+    with_length(ctx->n2, [&](auto NN) { Passes<T, decltype(NN)::value>::yfwd(ctx, w, s, A, B, np); });
+    with_length(ctx->n3, [&](auto NN) {
       Passes<T, decltype(NN)::value>::zfwd(ctx, w, s, np, A, c0, c2, f_dev, nstate, pair0, scale, acc ? 1 : 0);
     });
   }

@@ -4,9 +4,14 @@
 namespace mc {
 
 template struct Passes<double, 162>;
+template struct Passes<float, 162>;
 template struct Passes<double, 180>;
+template struct Passes<float, 180>;
 template struct Passes<double, 200>;
+template struct Passes<float, 200>;
 template struct Passes<double, 216>;
+template struct Passes<float, 216>;
 template struct Passes<double, 256>;
+template struct Passes<float, 256>;
 
 }  // namespace mc

@@ -4,8 +4,12 @@
 namespace mc {
 
 template struct Passes<double, 270>;
+template struct Passes<float, 270>;
 template struct Passes<double, 288>;
+template struct Passes<float, 288>;
 template struct Passes<double, 300>;
+template struct Passes<float, 300>;
 template struct Passes<double, 320>;
+template struct Passes<float, 320>;
 
 }  // namespace mc

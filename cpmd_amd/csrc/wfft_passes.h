@@ -378,9 +378,9 @@ __global__ __launch_bounds__(kThreads) void k_xvpsi(WParams w, v2<T>* __restrict
 // (256 VGPRs); FP32 keeps its register prefetch unconstrained
 #define F4_WAVES __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 1 : 2, 8)))
 
-template <int N>
+template <typename T, int N>
 struct F4Tile {
-  static constexpr int A = FastShape<N>::A, B = FastShape<N>::B;
+  static constexpr int A = Shape<T, N>::A, B = Shape<T, N>::B;
   static constexpr int G = A > B ? A : B;
   // lines per workgroup: a multiple of 4, so that the z runs of FP64 start on 64
   // bytes (108 x 120 x 160, 103 states, density: 649 us at 20 lines of the
@@ -389,16 +389,17 @@ struct F4Tile {
   static constexpr int kBuf = N * L;       // elements of one LDS buffer
 };
 
-// whether the engine of length N has the band structure (dft_band_in, dft16_band)
-template <int N>
-constexpr bool f4_band() { return FastShape<N>::A % 4 == 0 && FastShape<N>::A > 4; }
+// whether the engine of length N has the band structure (dft_band_in, dft16_band, stock_stages)
+template <typename T, int N>
+constexpr bool f4_band() { return Shape<T, N>::A % 4 == 0 && (Shape<T, N>::A > 4 || !four_step<T, N>()); }
 
-// LDS bytes of the fused kernels: the phase-1 twiddle table, with T3 (xvpsi)
-// the phase-3 table too, nb buffers, one int map of length N
+// LDS bytes of the fused kernels: the phase-1 twiddle table (the N-point table
+// itself for the engine of plan stages), with T3 (xvpsi) the phase-3 table too,
+// nb buffers, one int map of length N
 constexpr size_t kF4MaxLds = 98304;   // dynamic LDS the fused engine may take per workgroup
 template <typename T, int N, bool T3>
 constexpr size_t f4_lds(int nb) {
-  return sizeof(v2<T>) * (size_t)((T3 ? 2 : 1) * N + nb * F4Tile<N>::kBuf) + sizeof(int) * N;
+  return sizeof(v2<T>) * (size_t)((T3 && four_step<T, N>() ? 2 : 1) * N + nb * F4Tile<T, N>::kBuf) + sizeof(int) * N;
 }
 // Two buffers (one barrier less per transform) where they leave room for
 // enough workgroups: FP32 up to 64 KB; FP64, whose registers allow three to
@@ -406,6 +407,7 @@ constexpr size_t f4_lds(int nb) {
 // at 64 KB, i.e. two workgroups per CU)
 template <typename T, int N, bool T3>
 constexpr int f4_bufs() {
+  if (!four_step<T, N>()) return 2;   // the exchanges of xvpsi alternate between two
   return sizeof(T) == 4 ? (f4_lds<T, N, true>(2) <= 65536 ? 2 : 1) : (f4_lds<T, N, T3>(2) <= 40960 ? 2 : 1);
 }
 template <typename T, int N, bool T3>
@@ -450,7 +452,7 @@ __device__ __forceinline__ F4Bases f4_bases(int g, int l) {
 template <typename T, int N, bool T3>
 struct F4 {
   using V = v2<T>;
-  static constexpr int A = F4Tile<N>::A, B = F4Tile<N>::B, L = F4Tile<N>::L;
+  static constexpr int A = F4Tile<T, N>::A, B = F4Tile<T, N>::B, L = F4Tile<T, N>::L;
   static constexpr int NB = f4_bufs<T, N, T3>();
   static constexpr unsigned kNone = 0xffffffffu;
   V* t1;      // t1[k1 B + n2] = w^{n2 k1}, k1 < A, n2 < B (phase 1)
@@ -464,8 +466,8 @@ struct F4 {
     t1 = lds_base<T>();
     t3 = t1 + N;
     buf[0] = T3 ? t3 + N : t3;
-    buf[1] = NB == 2 ? buf[0] + F4Tile<N>::kBuf : buf[0];
-    map = reinterpret_cast<int*>(buf[0] + NB * F4Tile<N>::kBuf);
+    buf[1] = NB == 2 ? buf[0] + F4Tile<T, N>::kBuf : buf[0];
+    map = reinterpret_cast<int*>(buf[0] + NB * F4Tile<T, N>::kBuf);
     l = threadIdx.x % L;
     g = threadIdx.x / L;
     b12 = f4_bases<B, L>(g, l);
@@ -555,6 +557,80 @@ struct F4 {
   }
 };
 
+// The engine of plan stages with the interface of F4's phases 1 and 2: group g
+// of phase 1 holds x[B k + g] and runs the first stages, phase 2 group g runs the
+// others on the A-point results and ends with X(g + A k).  Its twiddles depend on
+// the group in phase 2 (in F4 in phase 1).  mid_put / mid_get move a line from
+// the second layout back to the first (xvpsi: V psi into the forward transform).
+template <typename T, int N>
+struct S4 {
+  using V = v2<T>;
+  static constexpr int A = F4Tile<T, N>::A, B = F4Tile<T, N>::B, L = F4Tile<T, N>::L;
+  static constexpr int NB = 2;
+  static constexpr unsigned kNone = 0xffffffffu;
+  V* tw;      // the N-point table
+  V* buf[2];
+  int* map;   // N ints after the buffers
+  int l, g;
+  F4Bases b12;
+
+  __device__ __forceinline__ void init(const double2* table) {
+    tw = lds_base<T>();
+    buf[0] = tw + N;
+    buf[1] = buf[0] + F4Tile<T, N>::kBuf;
+    map = reinterpret_cast<int*>(buf[1] + F4Tile<T, N>::kBuf);
+    l = threadIdx.x % L;
+    g = threadIdx.x / L;
+    b12 = f4_bases<B, L>(g, l);
+    load_tw<T>(tw, table, N);
+  }
+  __device__ __forceinline__ static V ld(const V* p, unsigned b) { return F4<T, N, false>::ld(p, b); }
+  __device__ __forceinline__ static void st(V* p, unsigned b, V v) { F4<T, N, false>::st(p, b, v); }
+  template <int K>
+  __device__ __forceinline__ static void fetch(const V* __restrict__ p, const unsigned (&off)[K], V (&r)[K]) {
+    F4<T, N, false>::fetch(p, off, r);
+  }
+  template <int K>
+  __device__ __forceinline__ static void store(V* __restrict__ p, const unsigned (&off)[K], const V (&r)[K]) {
+    F4<T, N, false>::store(p, off, r);
+  }
+  template <int DIR, bool PR = false>
+  __device__ __forceinline__ void phase1(V (&v)[A], V* bf) const {
+    if (g < B) {
+      stock_stages<N, 0, A, 1, 1, DIR, PR>(v, 0, tw);
+      V* w0 = bf + b12.wb[0];
+      V* w1 = bf + b12.wb[1];
+#pragma unroll
+      for (int k1 = 0; k1 < A; ++k1) ((k1 & 1) ? w1 : w0)[B * k1 * L] = v[k1];
+    }
+  }
+  template <int DIR>
+  __device__ __forceinline__ void phase2(V (&u)[B], const V* bf) const {
+    if (g < A) {
+      const V* r0 = bf + b12.rb[0];
+      const V* r1 = bf + b12.rb[1];
+#pragma unroll
+      for (int m = 0; m < B; ++m) u[m] = ((m & 1) ? r1 : r0)[m * L];
+      stock_stages<N, second_stage<N, A>(), B, 1, A, DIR, false>(u, g, tw);
+    }
+  }
+  __device__ __forceinline__ void mid_put(const V (&u)[B], V* bf) const {
+    if (g < A) {
+#pragma unroll
+      for (int k = 0; k < B; ++k) bf[(g + A * k) * L + l] = u[k];
+    }
+  }
+  __device__ __forceinline__ void mid_get(V (&v)[A], const V* bf) const {
+    if (g < B) {
+#pragma unroll
+      for (int k = 0; k < A; ++k) v[k] = bf[(B * k + g) * L + l];
+    }
+  }
+};
+
+template <typename T, int N, bool T3>
+using Engine = std::conditional_t<four_step<T, N>(), F4<T, N, T3>, S4<T, N>>;
+
 // ---------------------------------------------------------------------------
 // y pass, fused form: workgroup (column c, z tile, pairs p0 .. p0+ppb-1).
 // DIR=+1: sticks of column c in A -> B (dense y); DIR=-1: B -> sticks in A.
@@ -563,7 +639,7 @@ template <typename T, int N, int DIR, bool PR = false>
 __global__ __launch_bounds__(kThreads) F4_WAVES void k_ypass_f(WParams w, v2<T>* __restrict__ Ag, v2<T>* __restrict__ Bg,
                                                       int npairs, int ppb) {
   using V = v2<T>;
-  using X = F4<T, N, false>;
+  using X = Engine<T, N, false>;
   constexpr int A = X::A, B = X::B, L = X::L;
   X s;
   s.init(w.tw2);
@@ -653,7 +729,7 @@ __global__ __launch_bounds__(kThreads) F4_WAVES void k_xrho_f(WParams w, const v
                                                      int nstate, const double* __restrict__ f,
                                                      double* __restrict__ rho) {
   using V = v2<T>;
-  using X = F4<T, N, false>;
+  using X = Engine<T, N, false>;
   constexpr int A = X::A, B = X::B, L = X::L;
   X s;
   s.init(w.tw1);
@@ -705,8 +781,8 @@ __global__ __launch_bounds__(kThreads) F4_WAVES void k_xrho_f(WParams w, const v
   // read-modify-write of rho runs along x
   __syncthreads();
   double* stg = reinterpret_cast<double*>(s.buf[0]);
-  constexpr int LD = (sizeof(double) * L * (N + 1) <= sizeof(V) * X::NB * F4Tile<N>::kBuf) ? N + 1 : N;
-  static_assert(sizeof(double) * L * LD <= sizeof(V) * X::NB * F4Tile<N>::kBuf, "rho staging exceeds the buffers");
+  constexpr int LD = (sizeof(double) * L * (N + 1) <= sizeof(V) * X::NB * F4Tile<T, N>::kBuf) ? N + 1 : N;
+  static_assert(sizeof(double) * L * LD <= sizeof(V) * X::NB * F4Tile<T, N>::kBuf, "rho staging exceeds the buffers");
   if (s.g < A) {
 #pragma unroll
     for (int k = 0; k < B; ++k) stg[s.l * LD + s.g + A * k] = acc[k];
@@ -719,24 +795,28 @@ __global__ __launch_bounds__(kThreads) F4_WAVES void k_xrho_f(WParams w, const v
   }
 }
 
-// xvpsi, fused form (same contract as k_xvpsi): workgroup (z tile, y).  On
+// xvpsi, fused form (same contract as k_xvpsi): workgroup (z tile, y, run of
+// ppb pairs).  On
 // the FP32 path the next pair's loads are issued after phase kXPre.
 constexpr int kXPre = 1;
 template <typename T, int N, bool PR = false>
 __global__ __launch_bounds__(kThreads) F4_WAVES void k_xvpsi_f(WParams w, v2<T>* __restrict__ Bg, int npairs,
-                                                      const double* __restrict__ vpot) {
+                                                      int ppb, const double* __restrict__ vpot) {
   using V = v2<T>;
-  using X = F4<T, N, true>;
+  using X = Engine<T, N, true>;
   constexpr int A = X::A, B = X::B, L = X::L;
   X s;
   s.init(w.tw1);
   const int z0 = blockIdx.x * L, y = blockIdx.y;
   const int nz = min(L, w.n3 - z0);
+  // this workgroup's run of pairs
+  Bg += (size_t)blockIdx.z * ppb * ((size_t)w.ncols * w.n2 * w.n3);
+  npairs = min(ppb, npairs - (int)blockIdx.z * ppb);
   x_map(s, w, N);
   // V(r) of this tile, staged x-major (row stride L + 1) through buffer 2 so
   // that lane (l, g) picks up V(x = g + A k2, z0 + l) for its phase-2 values
   T* vst = reinterpret_cast<T*>(s.buf[1]);
-  static_assert(N * (L + 1) <= 2 * F4Tile<N>::kBuf, "V staging exceeds a buffer");
+  static_assert(N * (L + 1) <= 2 * F4Tile<T, N>::kBuf, "V staging exceeds a buffer");
   for (int e = threadIdx.x; e < L * N; e += kThreads) {
     const int zl = e / N, x = e - zl * N;
     vst[x * (L + 1) + zl] =
@@ -747,6 +827,43 @@ __global__ __launch_bounds__(kThreads) F4_WAVES void k_xvpsi_f(WParams w, v2<T>*
 #pragma unroll
   for (int k = 0; k < B; ++k) vr[k] = s.g < A ? vst[(s.g + A * k) * (L + 1) + s.l] : (T)0;
   if (X::NB == 1) __syncthreads();
+  if constexpr (!four_step<T, N>()) {
+    // the engine of plan stages: outputs x = g + A k, three exchanges over two
+    // alternating buffers (each is read behind a barrier before it is rewritten)
+    unsigned offi[A], offo[B];
+    x_offsets(s, w, y, z0, offi);
+    const bool act = s.g < A && z0 + s.l < w.n3;
+#pragma unroll
+    for (int k = 0; k < B; ++k) {
+      const int c = act ? s.map[s.g + A * k] : -1;
+      offo[k] = c >= 0 ? (unsigned)((((size_t)c * w.n2 + y) * w.n3 + z0 + s.l) * sizeof(V)) : X::kNone;
+    }
+    const size_t slab = (size_t)w.ncols * w.n2 * w.n3;
+    __syncthreads();   // V(r) is read out of the second buffer
+    V r[A];
+    if (npairs > 0) X::fetch(Bg, offi, r);
+    for (int pb = 0; pb < npairs; ++pb) {
+      V* Bs = Bg + (size_t)pb * slab;
+      V* b0 = s.buf[pb & 1];
+      V* b1 = s.buf[(pb & 1) ^ 1];
+      s.template phase1<1, PR>(r, b0);
+      if (pb + 1 < npairs) X::fetch(Bs + slab, offi, r);   // in flight through the rest of this pair
+      __syncthreads();
+      V u[B];
+      s.template phase2<1>(u, b0);
+#pragma unroll
+      for (int k = 0; k < B; ++k) u[k] = cscale(u[k], vr[k]);
+      s.mid_put(u, b1);
+      __syncthreads();
+      V v[A];
+      s.mid_get(v, b1);
+      s.template phase1<-1>(v, b0);
+      __syncthreads();
+      s.template phase2<-1>(u, b0);
+      X::store(Bs, offo, u);
+    }
+    return;
+  } else {
   unsigned off[A];
   x_offsets(s, w, y, z0, off);
   const size_t bslab = (size_t)w.ncols * w.n2 * w.n3;
@@ -782,6 +899,7 @@ __global__ __launch_bounds__(kThreads) F4_WAVES void k_xvpsi_f(WParams w, v2<T>*
     }
     if (X::NB == 1) __syncthreads();
   }
+  }   // four-step engine
 }
 
 // ---------------------------------------------------------------------------
@@ -904,7 +1022,7 @@ template <int DIR>
 void Passes<T, N>::ypass(mc_ctx* ctx, const WParams& w, const Shapes& s, V* A, V* B, int np) {
   const int kid = DIR > 0 ? MC_KID_YINV : MC_KID_YFWD;
   if constexpr (f4_ok<T, N>()) {
-    constexpr int L = F4Tile<N>::L;
+    constexpr int L = F4Tile<T, N>::L;
     const int zt = (ctx->n3 + L - 1) / L;
     // runs of pairs per (column, z tile): aimed at >= 65536 workgroups, i.e. a
     // few pairs per workgroup (at 192^3: 1.78 + 1.85 ms of y passes per CP
@@ -917,7 +1035,7 @@ void Passes<T, N>::ypass(mc_ctx* ctx, const WParams& w, const Shapes& s, V* A, V
       LAUNCH(kid, (k_ypass_f<T, N, DIR, PR>), dim3(ctx->ncols, zt, (np + ppb - 1) / ppb), dim3(kThreads),
              (f4_lds<T, N, false>()), w, A, B, np, ppb);
     };
-    if constexpr (DIR > 0 && f4_band<N>()) {
+    if constexpr (DIR > 0 && f4_band<T, N>()) {
       if (ctx->prune_y) go(std::true_type{});
       else go(std::false_type{});
     } else {
@@ -945,10 +1063,10 @@ void Passes<T, N>::xrho(mc_ctx* ctx, const WParams& w, const Shapes& s, const V*
     auto go = [&](auto PRC) {
       constexpr bool PR = decltype(PRC)::value;
       f4_allow_lds(&k_xrho_f<T, N, PR>, f4_lds<T, N, false>());
-      LAUNCH(MC_KID_XRHO, (k_xrho_f<T, N, PR>), dim3((ctx->n3 + F4Tile<N>::L - 1) / F4Tile<N>::L, ctx->n2),
+      LAUNCH(MC_KID_XRHO, (k_xrho_f<T, N, PR>), dim3((ctx->n3 + F4Tile<T, N>::L - 1) / F4Tile<T, N>::L, ctx->n2),
              dim3(kThreads), (f4_lds<T, N, false>()), w, B, np, pair0, nstate, f, rho);
     };
-    if constexpr (f4_band<N>()) {
+    if constexpr (f4_band<T, N>()) {
       if (ctx->prune_x) go(std::true_type{});
       else go(std::false_type{});
     } else {
@@ -967,10 +1085,17 @@ void Passes<T, N>::xvpsi(mc_ctx* ctx, const WParams& w, const Shapes& s, V* B, i
     auto go = [&](auto PRC) {
       constexpr bool PR = decltype(PRC)::value;
       f4_allow_lds(&k_xvpsi_f<T, N, PR>, f4_lds<T, N, true>());
-      LAUNCH(MC_KID_XVPSI, (k_xvpsi_f<T, N, PR>), dim3((ctx->n3 + F4Tile<N>::L - 1) / F4Tile<N>::L, ctx->n2),
-             dim3(kThreads), (f4_lds<T, N, true>()), w, B, np, vpot);
+      const int zt = (ctx->n3 + F4Tile<T, N>::L - 1) / F4Tile<T, N>::L;
+      // one run of all pairs (V(r) is staged once), or more where the mesh gives
+      // fewer than 1024 workgroups (80 x 64 x 60, 25 states, gradient in FP64: 89
+      // against 105 us; 80 x 144 x 96, 61 states, mixed: 392 against 422 us; runs
+      // for 4096 and more workgroups are slower at every mesh measured)
+      const int runs = std::max(1, std::min(np, 2047 / (zt * ctx->n2)));
+      const int ppb = (np + runs - 1) / runs;
+      LAUNCH(MC_KID_XVPSI, (k_xvpsi_f<T, N, PR>), dim3(zt, ctx->n2, (np + ppb - 1) / ppb), dim3(kThreads),
+             (f4_lds<T, N, true>()), w, B, np, ppb, vpot);
     };
-    if constexpr (f4_band<N>()) {
+    if constexpr (f4_band<T, N>()) {
       if (ctx->prune_x) go(std::true_type{});
       else go(std::false_type{});
     } else {
@@ -988,9 +1113,7 @@ void Passes<T, N>::xvpsi(mc_ctx* ctx, const WParams& w, const Shapes& s, V* B, i
   extern template struct Passes<double, n>; \
   extern template struct Passes<float, n>;
 MC_FAST_SIZES(MC_EXTERN_PASSES)
-#undef MC_EXTERN_PASSES
-#define MC_EXTERN_PASSES(n) extern template struct Passes<double, n>;
-MC_F64_SIZES(MC_EXTERN_PASSES)
+MC_MORE_SIZES(MC_EXTERN_PASSES)
 #undef MC_EXTERN_PASSES
 
 }  // namespace mc
