@@ -38,30 +38,38 @@ __global__ void k_fill(double* __restrict__ x, size_t n, double v) {
     x[i] = v;
 }
 
-// sum of x[0..n) into out[blockIdx.x]; fixed order for reproducibility
-__global__ __launch_bounds__(kThreads) void k_sum_partial(const double* __restrict__ x, size_t n,
-                                                          double* __restrict__ out) {
+// The sums that rhoofr reads back, in one launch and in a fixed order (one
+// thread per pair and sum took 33 us at 103 states on 108 x 120 x 160, this 4).  Workgroup
+// p < npairs: the zinv partials red[(p gx + b) 4 + k] of pair p, k = 0..3, into
+// out[4 p + k]; the other nsum workgroups: partial sums of rho[0..n) into out[4
+// npairs + ..].
+__global__ __launch_bounds__(kThreads) void k_rho_sums(const double* __restrict__ red, int gx, int npairs,
+                                                       const double* __restrict__ rho, size_t n, int nsum,
+                                                       double* __restrict__ out) {
+  __shared__ double part[kThreads];
+  if ((int)blockIdx.x < npairs) {
+    const int p = blockIdx.x, k = threadIdx.x & 3;
+    double s = 0.0;
+    for (int b = threadIdx.x >> 2; b < gx; b += kThreads / 4) s += red[((size_t)p * gx + b) * 4 + k];
+    part[threadIdx.x] = s;
+    __syncthreads();
+    for (int h = kThreads / 2; h >= 4; h >>= 1) {
+      if ((int)threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
+      __syncthreads();
+    }
+    if (threadIdx.x < 4) out[(size_t)p * 4 + threadIdx.x] = part[threadIdx.x];
+    return;
+  }
+  const int q = blockIdx.x - npairs;
   double s = 0.0;
-  for (size_t i = blockIdx.x * (size_t)kThreads + threadIdx.x; i < n; i += (size_t)gridDim.x * kThreads)
-    s += x[i];
+  for (size_t i = q * (size_t)kThreads + threadIdx.x; i < n; i += (size_t)nsum * kThreads) s += rho[i];
   s = warp_sum(s);
-  __shared__ double part[kThreads / 64];
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) {
     double t = 0.0;
-    for (int q = 0; q < kThreads / 64; ++q) t += part[q];
-    out[blockIdx.x] = t;
-  }
-}
-
-// per-pair sums of the zinv partials: red[(pair*gx + b)*4 + k] -> out[pair*4 + k]
-__global__ void k_reduce_pairs(const double* __restrict__ red, int gx, double* __restrict__ out) {
-  const int pair = blockIdx.x;
-  if (threadIdx.x < 4) {
-    double s = 0.0;
-    for (int b = 0; b < gx; ++b) s += red[((size_t)pair * gx + b) * 4 + threadIdx.x];
-    out[(size_t)pair * 4 + threadIdx.x] = s;
+    for (int v = 0; v < kThreads / 64; ++v) t += part[v];
+    out[(size_t)4 * npairs + q] = t;
   }
 }
 
@@ -173,7 +181,7 @@ static void rhoofr_impl(mc_ctx* ctx, const double2* c0, const double* f_host, in
   const WParams w = make_params(ctx);
   const Shapes s = shapes<T>(ctx);
   const int npairs = (nstate + 1) / 2;
-  const int nblk_sum = 1024;
+  const int nblk_sum = (int)std::min<size_t>(1024, (nnr1 + 2047) / 2048);
   WsUse use(ctx->w_a, ctx->w_b);
   ctx->keep_valid = false;
   V* K = keep ? keep_columns<T>(ctx, npairs) : nullptr;
@@ -192,8 +200,7 @@ static void rhoofr_impl(mc_ctx* ctx, const double2* c0, const double* f_host, in
   ctx->w_red.ensure(sizeof(double) * ((size_t)std::max(npairs, 1) * s.gx * 4 + (size_t)npairs * 4 + nblk_sum));
   double* red = ctx->w_red.as<double>();
   double* pair_sums = red + (size_t)std::max(npairs, 1) * s.gx * 4;
-  double* rsum_part = pair_sums + (size_t)npairs * 4;
-  LAUNCH(MC_KID_MISC, k_fill, dim3(1024), dim3(256), 0, rho, nnr1, 0.0);
+  if (npairs == 0) LAUNCH(MC_KID_MISC, k_fill, dim3(1024), dim3(256), 0, rho, nnr1, 0.0);
   V* A = ctx->w_a.as<V>();
   const size_t bslab = (size_t)ctx->n3 * ctx->ncols * ctx->n2;
   for (int pair0 = 0; pair0 < npairs; pair0 += P) {
@@ -204,7 +211,7 @@ static void rhoofr_impl(mc_ctx* ctx, const double2* c0, const double* f_host, in
     });
     with_length(ctx->n2, [&](auto NN) { Passes<T, decltype(NN)::value>::yinv(ctx, w, s, A, B, np); });
     with_length(ctx->n1, [&](auto NN) {
-      Passes<T, decltype(NN)::value>::xrho(ctx, w, s, B, np, pair0, nstate, ctx->w_f.as<double>(), rho);
+      Passes<T, decltype(NN)::value>::xrho(ctx, w, s, B, np, pair0, nstate, ctx->w_f.as<double>(), rho, pair0 == 0 ? 1 : 0);
     });
   }
   if (K) {   // the columns of every pair, for the next vpsi on these wavefunctions
@@ -214,8 +221,8 @@ static void rhoofr_impl(mc_ctx* ctx, const double2* c0, const double* f_host, in
     ctx->keep_tsize = (int)sizeof(T);
     ctx->keep_epoch = wfn_epoch();
   }
-  if (npairs > 0) LAUNCH(MC_KID_MISC, k_reduce_pairs, dim3(npairs), dim3(64), 0, red, s.gx, pair_sums);
-  LAUNCH(MC_KID_MISC, k_sum_partial, dim3(nblk_sum), dim3(kThreads), 0, rho, nnr1, rsum_part);
+  LAUNCH(MC_KID_MISC, k_rho_sums, dim3(npairs + nblk_sum), dim3(kThreads), 0, red, s.gx, npairs, rho, nnr1, nblk_sum,
+         pair_sums);
   std::vector<double> hs((size_t)npairs * 4 + nblk_sum);
   dl_add(ctx, hs.data(), pair_sums, sizeof(double) * hs.size());
   dl_finish(ctx);

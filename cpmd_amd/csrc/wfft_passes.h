@@ -220,16 +220,29 @@ __device__ __forceinline__ void put_cols(int ne, const int (&dst)[kMaxCol], cons
   __syncthreads();
 }
 
+// Zeros of the padding of rho that goes with the rows [y0, y0 + ny) of the
+// planes [z0, z0 + nz): the x padding, and behind the last row or plane the
+// padding rows and planes
+__device__ __forceinline__ void zero_padding(const WParams& w, double* __restrict__ rho, int y0, int ny, int z0,
+                                             int nz) {
+  const int y1 = y0 + ny == w.n2 ? w.kr2 : y0 + ny, z1 = z0 + nz == w.n3 ? w.kr3 : z0 + nz;
+  for (int z = z0; z < z1; ++z)
+    for (int y = y0; y < y1; ++y) {
+      const int x0 = y < w.n2 && z < w.n3 ? w.n1 : 0;
+      for (int x = x0 + threadIdx.x; x < w.kr1; x += kThreads) rho[(size_t)x + (size_t)w.kr1 * (y + (size_t)w.kr2 * z)] = 0.0;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // xrho: inverse x pass of every pair of the batch for one (z, y-tile) and
 // rho(r) += f1/omega Re(psi)^2 + f2/omega Im(psi)^2 (build_density_sum,
 // src/density_utils.mod.F90:61-80), accumulated in FP64; pairs with
-// f1 = f2 = 0 are skipped.
+// f1 = f2 = 0 are skipped.  first: rho is written (with its padding), not added to.
 // ---------------------------------------------------------------------------
 template <typename T, int N>
 __global__ __launch_bounds__(kThreads) void k_xrho(WParams w, const v2<T>* __restrict__ B, int npairs, int pair0,
                                                    int nstate, const double* __restrict__ f,
-                                                   double* __restrict__ rho, int ty) {
+                                                   double* __restrict__ rho, int ty, int first) {
   using V = v2<T>;
   const int n1 = N > 0 ? N : w.n1;
   V* tw = lds_base<T>();
@@ -280,9 +293,10 @@ __global__ __launch_bounds__(kThreads) void k_xrho(WParams w, const v2<T>* __res
     if (e < ne) {
       const int y = e / n1, x = e - y * n1;
       const size_t idx = (size_t)x + (size_t)w.kr1 * ((size_t)(y0 + y) + (size_t)w.kr2 * z);
-      rho[idx] += acc[k];
+      rho[idx] = first ? acc[k] : rho[idx] + acc[k];
     }
   }
+  if (first) zero_padding(w, rho, y0, ny, z, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -727,7 +741,7 @@ __device__ __forceinline__ void x_map(const X& s, const WParams& w, int n1) {
 template <typename T, int N, bool PR = false>
 __global__ __launch_bounds__(kThreads) F4_WAVES void k_xrho_f(WParams w, const v2<T>* __restrict__ Bg, int npairs, int pair0,
                                                      int nstate, const double* __restrict__ f,
-                                                     double* __restrict__ rho) {
+                                                     double* __restrict__ rho, int first) {
   using V = v2<T>;
   using X = Engine<T, N, false>;
   constexpr int A = X::A, B = X::B, L = X::L;
@@ -791,8 +805,9 @@ __global__ __launch_bounds__(kThreads) F4_WAVES void k_xrho_f(WParams w, const v
   for (int e = threadIdx.x; e < nz * N; e += kThreads) {
     const int zl = e / N, x = e - zl * N;
     const size_t idx = (size_t)x + (size_t)w.kr1 * ((size_t)y + (size_t)w.kr2 * (z0 + zl));
-    rho[idx] += stg[zl * LD + x];
+    rho[idx] = first ? stg[zl * LD + x] : rho[idx] + stg[zl * LD + x];
   }
+  if (first) zero_padding(w, rho, y, 1, z0, nz);
 }
 
 // xvpsi, fused form (same contract as k_xvpsi): workgroup (z tile, y, run of
@@ -994,7 +1009,7 @@ struct Passes {
   static void yinv(mc_ctx* ctx, const WParams& w, const Shapes& s, V* A, V* B, int np);
   static void yfwd(mc_ctx* ctx, const WParams& w, const Shapes& s, V* A, V* B, int np);
   static void xrho(mc_ctx* ctx, const WParams& w, const Shapes& s, const V* B, int np, int pair0, int nstate,
-                   const double* f, double* rho);
+                   const double* f, double* rho, int first);
   static void xvpsi(mc_ctx* ctx, const WParams& w, const Shapes& s, V* B, int np, const double* vpot);
   static void zfwd(mc_ctx* ctx, const WParams& w, const Shapes& s, int np, const V* A, const double2* c0, double2* c2,
                    const double* f, int nstate, int pair0, double scale, int acc);
@@ -1058,13 +1073,13 @@ void Passes<T, N>::yfwd(mc_ctx* ctx, const WParams& w, const Shapes& s, V* A, V*
 
 template <typename T, int N>
 void Passes<T, N>::xrho(mc_ctx* ctx, const WParams& w, const Shapes& s, const V* B, int np, int pair0, int nstate,
-                        const double* f, double* rho) {
+                        const double* f, double* rho, int first) {
   if constexpr (f4_ok<T, N>()) {
     auto go = [&](auto PRC) {
       constexpr bool PR = decltype(PRC)::value;
       f4_allow_lds(&k_xrho_f<T, N, PR>, f4_lds<T, N, false>());
       LAUNCH(MC_KID_XRHO, (k_xrho_f<T, N, PR>), dim3((ctx->n3 + F4Tile<T, N>::L - 1) / F4Tile<T, N>::L, ctx->n2),
-             dim3(kThreads), (f4_lds<T, N, false>()), w, B, np, pair0, nstate, f, rho);
+             dim3(kThreads), (f4_lds<T, N, false>()), w, B, np, pair0, nstate, f, rho, first);
     };
     if constexpr (f4_band<T, N>()) {
       if (ctx->prune_x) go(std::true_type{});
@@ -1075,7 +1090,7 @@ void Passes<T, N>::xrho(mc_ctx* ctx, const WParams& w, const Shapes& s, const V*
   } else {
     const size_t sh = sizeof(V) * (size_t)ctx->n1 * (1 + s.ty);
     LAUNCH(MC_KID_XRHO, (k_xrho<T, N>), dim3((ctx->n2 + s.ty - 1) / s.ty, ctx->n3), dim3(kThreads), sh, w, B, np,
-           pair0, nstate, f, rho, s.ty);
+           pair0, nstate, f, rho, s.ty, first);
   }
 }
 
