@@ -255,21 +255,26 @@ __global__ __launch_bounds__(256, 2) void k_tn_f64(const double* __restrict__ A,
 // and imaginary part of one coefficient: two MFMA row blocks.  A's columns are
 // copied straight to LDS (1 KiB each); G goes through registers, its 16-byte
 // loads only where GV (even leading dimension, aligned).  M even; lda, ldd
-// even and A, D 16-byte aligned.
+// even and A, D 16-byte aligned.  INPL (D is A; G upper triangular, or all of n
+// in one tile): a workgroup takes the column tiles of its rows from the last to
+// the first, so that no column is written before every product that reads it.
 // ---------------------------------------------------------------------------
-template <int NJ, bool PROJ, bool GV>
-__global__ __launch_bounds__(256, 2) void k_nn_f64(const double* __restrict__ A, int lda,
+template <int NJ, bool PROJ, bool GV, bool INPL>
+__global__ __launch_bounds__(256, 2) void k_nn_f64(const double* A, int lda,
                                                    const double* __restrict__ G, int ldgm, int M, int k, int n,
-                                                   double alpha, double beta, double* __restrict__ D, int ldd,
+                                                   double alpha, double beta, double* D, int ldd,
                                                    int upper_g, FnlEpi epi, ProjTab proj, int tn, int total) {
   constexpr int TI = 128, TJ = 32 * NJ;
   constexpr int kStageA = kKs * TI * 8, kStage = kStageA + TJ * 128;
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kStage];
   const int t = xcd_index(total);
   if (t >= total) return;
-  const int rt = t / tn, ct = t - rt * tn;
-  const int i0 = rt * TI, j0 = ct * TJ;
+  const int rt = INPL ? t : t / tn;
+  const int i0 = rt * TI;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  for (int ct = INPL ? tn - 1 : t - rt * tn, left = INPL ? tn : 1; left > 0; --ct, --left) {
+  if (INPL && left < tn) __syncthreads();   // the stages are free again
+  const int j0 = ct * TJ;
   const int kmax = upper_g ? min(k, j0 + TJ) : k;
   // A: wave w copies the columns w, w + 4, ... of a slice; lane -> rows 2 lane,
   // 2 lane + 1.  Rows beyond M repeat the last pair: they are not stored.
@@ -446,6 +451,7 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(const double* __restrict__ A,
       }
     }
   }
+  }   // column tiles
 }
 
 // Cost of an edge of n in tiles of 32 w: the padded edge, narrow tiles
@@ -563,23 +569,29 @@ bool nn_f64_form(const double* A, int lda, int M, const double* D, int ldd, cons
          (!epi || aligned16(epi->vcm));
 }
 
+bool nn_f64_in_place(int n, bool upper_g) { return upper_g || n <= 32 * tile_width(n, 1, 5); }
+
 void nn_f64(mc_ctx* ctx, const double* A, int lda, const double* G, int ldgm, int M, int k, int n, double alpha,
             double beta, double* D, int ldd, bool upper_g, const FnlEpi& epi, const ProjTab* proj, int kid) {
   const int nj = tile_width(n, 1, 5);
   const int tm = (M + 127) / 128, tn = (n + 32 * nj - 1) / (32 * nj);
-  const int total = tm * tn, launch = (total + kXcds - 1) / kXcds * kXcds;
+  const bool inpl = D == A;
+  MC_CHECK(!inpl || nn_f64_in_place(n, upper_g), MC_ERR_INTERNAL, "A G in place needs an upper G or one column tile");
+  const int total = inpl ? tm : tm * tn, launch = (total + kXcds - 1) / kXcds * kXcds;
   const bool gv = ldgm % 2 == 0 && aligned16(G);
   const ProjTab pt = proj ? *proj : ProjTab{};
   timer_begin(ctx, kid);
-#define MC_NN(NJ, PR, GV)                                                                                     \
-  hipLaunchKernelGGL((k_nn_f64<NJ, PR, GV>), dim3(launch), dim3(256), 0, ctx->stream, A, lda, G, ldgm, M, k, n, \
+#define MC_NN(NJ, PR, GV, IP)                                                                                 \
+  hipLaunchKernelGGL((k_nn_f64<NJ, PR, GV, IP>), dim3(launch), dim3(256), 0, ctx->stream, A, lda, G, ldgm, M, k, n, \
                      alpha, beta, D, ldd, upper_g ? 1 : 0, epi, pt, tn, total)
-#define MC_NN_J(NJ)                          \
-  do {                                       \
-    if (proj && gv) MC_NN(NJ, true, true);   \
-    else if (proj) MC_NN(NJ, true, false);   \
-    else if (gv) MC_NN(NJ, false, true);     \
-    else MC_NN(NJ, false, false);            \
+#define MC_NN_J(NJ)                                    \
+  do {                                                 \
+    if (proj && gv) MC_NN(NJ, true, true, false);      \
+    else if (proj) MC_NN(NJ, true, false, false);      \
+    else if (inpl && gv) MC_NN(NJ, false, true, true); \
+    else if (inpl) MC_NN(NJ, false, false, true);      \
+    else if (gv) MC_NN(NJ, false, true, false);        \
+    else MC_NN(NJ, false, false, false);               \
   } while (0)
   switch (nj) {
     case 1: MC_NN_J(1); break;

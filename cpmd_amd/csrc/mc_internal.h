@@ -419,6 +419,11 @@ int tn_f64_partials(mc_ctx* ctx, const double* A, int lda, const double* B, int 
 bool nn_f64_form(const double* A, int lda, int M, const double* D, int ldd, const FnlEpi* epi);
 void nn_f64(mc_ctx* ctx, const double* A, int lda, const double* G, int ldgm, int M, int k, int n, double alpha,
             double beta, double* D, int ldd, bool upper_g, const FnlEpi& epi, const ProjTab* proj, int kid);
+// whether nn_f64 may run with D = A
+bool nn_f64_in_place(int n, bool upper_g);
+// U^T U = S (upper triangle of S in place) and X = U^-1 (n x n, W scratch n x n);
+// info (device): 0 or the order of the first leading minor that is not positive (chol.hip)
+void chol_inverse(mc_ctx* ctx, double* S, int n, double* X, double* W, int* info);
 // fnl (v0 = 0, first variant) and dfnl from the partials of the projector operand
 void reduce_proj(mc_ctx* ctx, int nsplit, const ProjTab& t, int nv, int n, int nat, int nhxs, double tpiba,
                  double* fnl, double* dfnl);

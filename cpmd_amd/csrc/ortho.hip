@@ -11,9 +11,8 @@
 //   fnonloc   src/fnonloc_utils.mod.F90:209-303    c2 += -f (-i)^l twnl sum_ia eigr dd
 //
 // Dense n x n factorisations stay in FP64 on the GPU:
-//  * Cholesky (upper, LAPACK dpotrf semantics) is a left-looking column sweep
-//    in one workgroup; the triangular inverse (dtrtri) solves the columns of
-//    U X = I in parallel, one wavefront per column;
+//  * the Cholesky factor (upper, LAPACK dpotrf semantics) and its inverse are
+//    blocked (chol.hip);
 //  * Loewdin's S^-1/2 is obtained with the coupled Newton-Schulz iteration
 //    (Higham, "Functions of Matrices", 2008, eq. 6.35) on MFMA, which converges
 //    to the same unique SPD inverse square root that CPMD assembles from the
@@ -31,145 +30,6 @@ namespace mc {
 // ---------------------------------------------------------------------------
 // small kernels
 // ---------------------------------------------------------------------------
-
-// Cholesky S = U^T U of the upper triangle of S (n x n, column-major lds) in
-// place, blocked right-looking with 64-wide blocks; the lower triangle is set
-// to zero.  info (device) = 0 or the order of the first non-positive leading
-// minor (dpotrf); once set, the later launches return at once.
-constexpr int kPb = 64;
-
-// factor the diagonal block S(kb:kb+nb, kb:kb+nb) in LDS, right-looking
-__global__ __launch_bounds__(256) void k_potrf_diag(double* __restrict__ S, int lds, int kb, int nb, int* info) {
-  __shared__ double T[kPb][kPb + 1];
-  __shared__ int bad;
-  if (kb > 0 && *info) return;
-  const int t = threadIdx.x;
-  for (int e = t; e < nb * nb; e += 256) {
-    const int r = e % nb, c = e / nb;
-    T[r][c] = S[(kb + r) + (size_t)lds * (kb + c)];
-  }
-  if (t == 0) bad = 0;
-  __syncthreads();
-  for (int j = 0; j < nb; ++j) {
-    if (t == 0) {
-      const double d = T[j][j];
-      if (!(d > 0.0)) bad = kb + j + 1;
-      else T[j][j] = sqrt(d);
-    }
-    __syncthreads();
-    if (bad) break;
-    const double dj = T[j][j];
-    for (int c = j + 1 + t; c < nb; c += 256) T[j][c] /= dj;
-    __syncthreads();
-    const int m = nb - j - 1;   // trailing (r, c), j < r <= c < nb
-    for (int e = t; e < m * m; e += 256) {
-      const int r = j + 1 + e % m, c = j + 1 + e / m;
-      if (r <= c) T[r][c] -= T[j][r] * T[j][c];
-    }
-    __syncthreads();
-  }
-  for (int e = t; e < nb * nb; e += 256) {
-    const int r = e % nb, c = e / nb;
-    if (r <= c) S[(kb + r) + (size_t)lds * (kb + c)] = T[r][c];
-  }
-  if (t == 0 && (bad || kb == 0)) *info = bad;
-}
-
-// block row: U(kb:kb+nb, j) = U_kk^-T S(kb:kb+nb, j) for kb+nb <= j < n; one
-// thread per column, forward substitution with the column staged in LDS
-__global__ __launch_bounds__(64) void k_potrf_trsm(double* __restrict__ S, int lds, int n, int kb, int nb,
-                                                   const int* info) {
-  __shared__ double U[kPb][kPb + 1];
-  __shared__ double y[kPb][kPb + 1];
-  if (*info) return;
-  const int t = threadIdx.x;
-  for (int e = t; e < nb * nb; e += 64) {
-    const int r = e % nb, c = e / nb;
-    U[r][c] = S[(kb + r) + (size_t)lds * (kb + c)];
-  }
-  const int j = kb + nb + blockIdx.x * 64 + t;
-  if (j < n)
-    for (int r = 0; r < nb; ++r) y[r][t] = S[(kb + r) + (size_t)lds * j];
-  __syncthreads();
-  if (j >= n) return;
-  for (int r = 0; r < nb; ++r) {
-    double v = y[r][t];
-    for (int k = 0; k < r; ++k) v -= U[k][r] * y[k][t];
-    y[r][t] = v / U[r][r];
-  }
-  for (int r = 0; r < nb; ++r) S[(kb + r) + (size_t)lds * j] = y[r][t];
-}
-
-// trailing update S(i, j) -= sum_k U(k, i) U(k, j), k in the block row,
-// kb+nb <= i <= j < n, 32 x 32 tiles (upper tiles only)
-__global__ __launch_bounds__(256) void k_potrf_update(double* __restrict__ S, int lds, int n, int kb, int nb,
-                                                      const int* info) {
-  __shared__ double A[kPb][33];
-  __shared__ double B[kPb][33];
-  if (*info) return;
-  const int ti = blockIdx.x, tj = blockIdx.y;
-  if (ti > tj) return;
-  const int i0 = kb + nb + 32 * ti, j0 = kb + nb + 32 * tj;
-  const int t = threadIdx.x;
-  for (int e = t; e < nb * 32; e += 256) {
-    const int k = e % nb, c = e / nb;
-    A[k][c] = i0 + c < n ? S[(kb + k) + (size_t)lds * (i0 + c)] : 0.0;
-    B[k][c] = j0 + c < n ? S[(kb + k) + (size_t)lds * (j0 + c)] : 0.0;
-  }
-  __syncthreads();
-  for (int e = t; e < 32 * 32; e += 256) {
-    const int r = e % 32, c = e / 32;
-    const int i = i0 + r, j = j0 + c;
-    if (i >= n || j >= n || i > j) continue;
-    double s = 0.0;
-    for (int k = 0; k < nb; ++k) s += A[k][r] * B[k][c];
-    S[i + (size_t)lds * j] -= s;
-  }
-}
-
-__global__ void k_zero_lower(double* __restrict__ S, int n, int lds) {
-  const int j = blockIdx.x;
-  for (int i = j + 1 + threadIdx.x; i < n; i += blockDim.x) S[i + (size_t)lds * j] = 0.0;
-}
-
-static void potrf_upper_dev(mc_ctx* ctx, double* S, int n, int lds, int* info) {
-  for (int kb = 0; kb < n; kb += kPb) {
-    const int nb = std::min(kPb, n - kb), rest = n - kb - nb;
-    hipLaunchKernelGGL(k_potrf_diag, dim3(1), dim3(256), 0, ctx->stream, S, lds, kb, nb, info);
-    MC_HIP(hipGetLastError());
-    if (rest <= 0) break;
-    hipLaunchKernelGGL(k_potrf_trsm, dim3((rest + 63) / 64), dim3(64), 0, ctx->stream, S, lds, n, kb, nb, info);
-    MC_HIP(hipGetLastError());
-    const int nt = (rest + 31) / 32;
-    hipLaunchKernelGGL(k_potrf_update, dim3(nt, nt), dim3(256), 0, ctx->stream, S, lds, n, kb, nb, info);
-    MC_HIP(hipGetLastError());
-  }
-  hipLaunchKernelGGL(k_zero_lower, dim3(n), dim3(256), 0, ctx->stream, S, n, lds);
-  MC_HIP(hipGetLastError());
-}
-
-// X = U^{-1} (upper): one 64-thread workgroup per column j solves U x = e_j
-// by back substitution with x staged in LDS (n doubles).
-__global__ __launch_bounds__(64) void k_trtri_upper(const double* __restrict__ U, int n, int ldu,
-                                                    double* __restrict__ X, int ldx) {
-  extern __shared__ double xs[];
-  const int j = blockIdx.x;
-  const int l = threadIdx.x;
-  for (int i = l; i < n; i += 64) xs[i] = 0.0;
-  __syncthreads();
-  if (l == 0) xs[j] = 1.0 / U[j + (size_t)ldu * j];
-  __syncthreads();
-  for (int i = j - 1; i >= 0; --i) {
-    double s = 0.0;
-    for (int k = i + 1 + l; k <= j; k += 64) s += U[i + (size_t)ldu * k] * xs[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-    if (l == 0) xs[i] = -s / U[i + (size_t)ldu * i];
-    __syncthreads();
-  }
-  double* x = X + (size_t)ldx * j;
-  for (int i = l; i < n; i += 64) x[i] = xs[i];
-}
 
 // a(i,j) *= f(i) f(j) with f = (occupation != 0) (gscal, forces_driver.mod.F90:502-518)
 __global__ void k_gscal(double* __restrict__ a, int n, int lda, const double* __restrict__ focc) {
@@ -373,10 +233,16 @@ void ovlap_dev(mc_ctx* ctx, int n, double* a_dev, int lda, const double2* c1, co
           ctx->geq0 != 0, c1 == c2, a_dev, lda, nullptr);
 }
 
-// C <- C X with X (n x n) on the device; through the workspace copy of C.  With
+// C <- C X with X (n x n) on the device; in place in FP64 where the product allows
+// it (X upper, or few states), else through the workspace copy of C.  With
 // split-bf16 products C X is formed as C + C (X - I), so that the rounding of the
 // product scales with |X - I| (small near orthonormality), not with |X|.
 static void apply_right(mc_ctx* ctx, double2* c, const double* X, int n, bool upper) {
+  const int ld = wfn_ld(ctx);
+  if (!ctx->gemm_x3 && nn_f64_in_place(n, upper) && nn_f64_form((const double*)c, ld, ld, (const double*)c, ld, nullptr)) {
+    nn_f64(ctx, (const double*)c, ld, X, n, ld, n, n, 1.0, 0.0, (double*)c, ld, upper, FnlEpi{}, nullptr, MC_KID_GEMM);
+    return;
+  }
   const size_t bytes = sizeof(double2) * (size_t)ctx->ldg * n;
   ctx->w_wfn.ensure(bytes);
   MC_HIP(hipMemcpyAsync(ctx->w_wfn.p, c, bytes, hipMemcpyDeviceToDevice, ctx->stream));
@@ -406,14 +272,12 @@ void rgs_dev(mc_ctx* ctx, double2* c, int n, double* smat_host) {
   double* X = small(ctx, 1, n);
   ovlap_dev(ctx, n, S, n, c, c);
   ctx->w_info.ensure(sizeof(int));
-  potrf_upper_dev(ctx, S, n, n, ctx->w_info.as<int>());
+  chol_inverse(ctx, S, n, X, small(ctx, 2, n), ctx->w_info.as<int>());
   int info = 0;
   MC_HIP(hipMemcpyAsync(&info, ctx->w_info.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   MC_HIP(hipStreamSynchronize(ctx->stream));
   MC_CHECK(info == 0, MC_ERR_NOTPOSDEF,
            "UINV| the leading minor of order " + std::to_string(info) + " is not positive definite");
-  hipLaunchKernelGGL(k_trtri_upper, dim3(n), dim3(64), sizeof(double) * n, ctx->stream, S, n, n, X, n);
-  MC_HIP(hipGetLastError());
   apply_right(ctx, c, X, n, true);
   zclean(ctx, c, n);
   if (smat_host) {
