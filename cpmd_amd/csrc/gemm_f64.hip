@@ -7,8 +7,8 @@
 //             A optionally the projectors (fnonloc).
 //
 // A workgroup of 4 waves (2 x 2) computes 32 NI x 32 NJ of the result, a wave
-// 16 NI x 16 NJ of it; the tile edges follow the result's (tile_width), so
-// that 130 states take one 160-wide tile and not two of 128.  K advances in
+// 16 NI x 16 NJ of it; the tile edges follow the result's (tile_width,
+// nn_width).  K advances in
 // slices of 16 through two LDS stages.  Both operands of a slice are copied
 // straight to LDS 16 bytes per lane (global_load_lds_dwordx4), in 1 KiB runs
 // that cover whole 128-byte lines, while the slice before is multiplied.  Both
@@ -23,7 +23,8 @@
 // before the first read of every slice.
 //
 // Contraction order: the k pairs of a 16-byte chunk go to consecutive MFMAs
-// (lane group q holds k = 8h + 2q + s in step (h, s)), for A and B alike.
+// (lane group q holds k = 8h + 2q + s in step (h, s)), for A and B alike; A G
+// stages G so that they are k = 8h + 4s + q.
 //
 // MFMA operand layout (16x16x4 f64, checked on gfx950 with a lane probe):
 // lane l holds A[i = l%16][k = l/16], B[k = l/16][j = l%16] and, in
@@ -303,7 +304,9 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(const double* A, int lda,
         *reinterpret_cast<d2*>(sa + (wave + 4 * u) * 1024 + lane * 16) = proj_value(Raw{ea[u], ta[u], 0.0}, la[u], false);
     }
   };
-  // G: thread -> column t/8 + 32 u of the tile, chunk t%8
+  // G: thread -> column t/8 + 32 u of the tile, k = 2 (t%8), + 1 of the slice.  Chunk
+  // 4 h + q holds k = 8 h + q, 8 h + 4 + q: a 16-byte read feeds two instructions that
+  // take four successive k each, the order of k_gemm_nn (same bits).
   const int gc = threadIdx.x >> 3, gq = threadIdx.x & 7;
   d2 rg[NJ];
   auto fetch_g = [&](int kb) {   // a whole slice; columns beyond n repeat the last one (not stored)
@@ -317,7 +320,12 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(const double* A, int lda,
   auto put_g = [&](int st) {
     unsigned char* sg = lds + st * kStage + kStageA;
 #pragma unroll
-    for (int u = 0; u < NJ; ++u) *reinterpret_cast<d2*>(sg + 16 * chunk_slot(gc + 32 * u, gq)) = rg[u];
+    for (int u = 0; u < NJ; ++u) {
+      double* d = reinterpret_cast<double*>(sg) + ((gq >> 1) & 1);
+      const int q = (gq & 4) + 2 * (gq & 1);
+      d[2 * chunk_slot(gc + 32 * u, q)] = rg[u].x;
+      d[2 * chunk_slot(gc + 32 * u, q + 1)] = rg[u].y;
+    }
   };
   const int wr = (wave >> 1) * 64, wc = (wave & 1) * 16 * NJ;
   const int li = lane & 15, lq = lane >> 4;
@@ -339,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(const double* A, int lda,
         fg[b] = *reinterpret_cast<const d2*>(sg + 16 * chunk_slot(wc + 16 * b + li, 4 * h + lq));
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
-        const int kk = 8 * h + 2 * lq + s;
+        const int kk = 8 * h + 4 * s + lq;
         d2 fa[2];
 #pragma unroll
         for (int a = 0; a < 2; ++a)
@@ -467,6 +475,21 @@ int tile_width(int n, int least, int most) {
   return best;
 }
 
+// Column tiles of A G out of place, 32 or 64 wide: the workgroups of wider ones
+// fill the registers and LDS of a CU in twos, and nothing runs beside the first
+// copies and the store of a tile, which count with the short K of most products
+// here.  64 where there are 8 such tiles for each CU and the padding allows it.
+// Widths 32, 64, 96, 128, 160 at M x k x n, us:
+//   396,408 x 512 x 512   3628  3409  4037  3654  4462
+//   136,700 x 512 x 130    232   258   272   348   300   (projectors)
+//    26,100 x 386 x 512    198   227   252   231   275
+//    13,050 x 512 x 386    115   111   113   145   171
+//     1,900 x 128 x 128     16    17    22    27    32
+int nn_width(int tm, int n) {
+  const int w1 = (n + 31) / 32, w2 = (n + 63) / 64;
+  return tm * (long long)w2 >= 2048 && w2 * 64 * 1.06 <= w1 * 32 * 1.12 ? 2 : 1;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <int NI, int NJ>
@@ -573,9 +596,10 @@ bool nn_f64_in_place(int n, bool upper_g) { return upper_g || n <= 32 * tile_wid
 
 void nn_f64(mc_ctx* ctx, const double* A, int lda, const double* G, int ldgm, int M, int k, int n, double alpha,
             double beta, double* D, int ldd, bool upper_g, const FnlEpi& epi, const ProjTab* proj, int kid) {
-  const int nj = tile_width(n, 1, 5);
-  const int tm = (M + 127) / 128, tn = (n + 32 * nj - 1) / (32 * nj);
   const bool inpl = D == A;
+  const int tm = (M + 127) / 128;
+  const int nj = inpl ? tile_width(n, 1, 5) : nn_width(tm, n);
+  const int tn = (n + 32 * nj - 1) / (32 * nj);
   MC_CHECK(!inpl || nn_f64_in_place(n, upper_g), MC_ERR_INTERNAL, "A G in place needs an upper G or one column tile");
   const int total = inpl ? tm : tm * tn, launch = (total + kXcds - 1) / kXcds * kXcds;
   const bool gv = ldgm % 2 == 0 && aligned16(G);
@@ -584,23 +608,32 @@ void nn_f64(mc_ctx* ctx, const double* A, int lda, const double* G, int ldgm, in
 #define MC_NN(NJ, PR, GV, IP)                                                                                 \
   hipLaunchKernelGGL((k_nn_f64<NJ, PR, GV, IP>), dim3(launch), dim3(256), 0, ctx->stream, A, lda, G, ldgm, M, k, n, \
                      alpha, beta, D, ldd, upper_g ? 1 : 0, epi, pt, tn, total)
+#define MC_NN_I(NJ)                            \
+  do {                                         \
+    if (gv) MC_NN(NJ, false, true, true);      \
+    else MC_NN(NJ, false, false, true);        \
+  } while (0)
 #define MC_NN_J(NJ)                                    \
   do {                                                 \
     if (proj && gv) MC_NN(NJ, true, true, false);      \
     else if (proj) MC_NN(NJ, true, false, false);      \
-    else if (inpl && gv) MC_NN(NJ, false, true, true); \
-    else if (inpl) MC_NN(NJ, false, false, true);      \
     else if (gv) MC_NN(NJ, false, true, false);        \
     else MC_NN(NJ, false, false, false);               \
   } while (0)
-  switch (nj) {
-    case 1: MC_NN_J(1); break;
-    case 2: MC_NN_J(2); break;
-    case 3: MC_NN_J(3); break;
-    case 4: MC_NN_J(4); break;
-    default: MC_NN_J(5); break;
+  if (!inpl) {
+    if (nj == 1) MC_NN_J(1);
+    else MC_NN_J(2);
+  } else {
+    switch (nj) {
+      case 1: MC_NN_I(1); break;
+      case 2: MC_NN_I(2); break;
+      case 3: MC_NN_I(3); break;
+      case 4: MC_NN_I(4); break;
+      default: MC_NN_I(5); break;
+    }
   }
 #undef MC_NN_J
+#undef MC_NN_I
 #undef MC_NN
   MC_HIP(hipGetLastError());
   timer_end(ctx, kid);

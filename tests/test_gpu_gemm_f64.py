@@ -61,6 +61,23 @@ def test_rotate_edges(gpu, n):
             assert np.all(np.abs(getattr(out, part) - ref) <= 2 * (n + 8) * U * mag)
 
 
+@pytest.mark.parametrize("n", [250, 256])
+def test_rotate_wide_tiles(gpu, n):
+    """Enough rows for the 64-wide tiles (2048 of them), odd rows left over."""
+    sysm = S.make_system(30.0, 1, 30.0, nstate=1)
+    assert (2 * sysm.gset.ngw + 127) // 128 * 4 >= 2048
+    a, b = _wfn(sysm, n, 3), _wfn(sysm, n, 4)
+    g = np.random.default_rng(5).standard_normal((n, n))
+    out = ops.Context(sysm.cell, sysm.gset).rotate(1.5, a, -0.75, b, g)
+    rows = np.r_[0:sysm.gset.ngw:97, sysm.gset.ngw - 70:sysm.gset.ngw]
+    lg = g.astype(np.longdouble)
+    for part in ("real", "imag"):
+        la, lb = getattr(a, part)[rows].astype(np.longdouble), getattr(b, part)[rows].astype(np.longdouble)
+        ref = 1.5 * (la @ lg) - 0.75 * lb
+        mag = (1.5 * (np.abs(la) @ np.abs(lg)) + 0.75 * np.abs(lb)).astype(np.float64)
+        assert np.all(np.abs(getattr(out, part)[rows] - ref) <= 2 * (n + 8) * U * mag)
+
+
 @pytest.mark.parametrize("na,n", [((1, 0), 1), ((3, 5), 17), ((0, 7), 64), ((21, 44), 33)])
 def test_stacked_projectors(gpu, sysm, na, n):
     """fnl, dfnl and fnonloc over several species and projectors (l = 0 .. 3, a
