@@ -228,11 +228,14 @@ struct DensitySet {
   DevBuf d_gm, d_gidx, d_scg, d_gk;
   DevBuf d_sp_start, d_sp_of, d_zv, d_raggio, d_vps, d_rhops;
   DevBuf d_tau, d_ph1, d_ph2, d_ph3;   // d_tau: [tau (3, nat) | fractional coordinates (3, nat)]
-  DevBuf w_W, w_g, w_part;
-  // z-sticks of the density set: the distinct (m1, m2) (d_stk, sorted) and
-  // the stick of each G (d_sidx); operands of the stick GEMMs of vofrho
-  int nstick = 0;
-  DevBuf d_stk, d_sidx;
+  DevBuf w_W, w_V, w_part;
+  std::vector<int> gperm;   // device order of the G's -> the caller's (vofrho.hip)
+  // z-sticks of the density set: the distinct (m1, m2) (d_stk, m1 fastest) and
+  // the stick of each G (d_sidx); G_k = base_k(stick) + m3 b3_k (nby = 2); operands
+  // of the stick GEMMs of vofrho
+  int nstick = 0, nby = 2;
+  double b3[3] = {};
+  DevBuf d_stk, d_sidx, d_base;
   DevBuf w_q, w_bs, w_bf, w_sf, w_y, w_t;
 };
 

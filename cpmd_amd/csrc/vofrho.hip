@@ -1,13 +1,19 @@
 // The density -> potential step on gfx950 (vofrhoa + vofrhob, closed shell,
 // LDA) and the Ewald real-space sum, all FP64:
 //
+//   structure factors of the z-sticks as a GEMM over the atoms
 //   rho(r) --x,y,z forward passes--> W = N rho(G)        (dense mesh, fwfftn)
-//   per G (thread per G, loop over atoms with per-atom phase tables):
-//       eivps, eirop (eicalc), vtemp and the ppener energy sums
-//   W <- 0; W(+-G) = vtemp, conj(vtemp)
-//   per G x atom block: potfor partial forces, reduced in a fixed order
-//   W --z,y,x inverse passes--> v(r) = Re W + V_xc(rho(r)), E_xc sums (fused
+//   per G: eivps, eirop (eicalc), the ppener energy sums, W2(+-G) = vtemp,
+//       conj(vtemp) and the stick operand of potfor
+//   potfor as a GEMM over the sticks, forces reduced in a fixed order
+//   W2 --z,y,x inverse passes--> v(r) = Re W2 + V_xc(rho(r)), E_xc sums (fused
 //   into the last x pass)
+//
+// The density G's are kept in the order (m3, m2, m1), m1 fastest, with the
+// sticks in the order (m2, m1): neighbouring G's are neighbours on the mesh and
+// among the sticks, so that the per-G pass reads and writes whole lines (in
+// CPMD's order of |G|^2, i.e. scattered, three kernels took 325 us at 192^3 / 1.6M
+// G's, now one takes 48).
 //
 // References: vofrhoa src/vofrhoa_utils.mod.F90:41-144 (fwfftn :92, potfor
 // :101, ppener :103-122), eicalc src/eicalc_utils.mod.F90:33-173, ppener
@@ -182,17 +188,12 @@ __global__ __launch_bounds__(kThreads) void k_dx_inv_xc(DParams d, const double2
       v[idx] = 0.0;
     }
   }
+  // padding rows and planes behind the last ones
+  const int y1 = y0 + ny == d.n2 ? d.kr2 : y0 + ny, z1 = z + 1 == d.n3 ? d.kr3 : z + 1;
+  for (int zz = z; zz < z1; ++zz)
+    for (int yy = zz < d.n3 ? y0 + ny : y0; yy < y1; ++yy)
+      for (int x = threadIdx.x; x < d.kr1; x += kThreads) v[(size_t)x + (size_t)d.kr1 * (yy + (size_t)d.kr2 * zz)] = 0.0;
   block_sum_store<2>(acc, part + 2 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x), 2);
-}
-
-// zero the padding planes y >= n2 and z >= n3 of v (the x passes write y < n2, z < n3)
-__global__ void k_pad_zero(double* __restrict__ v, int n2, int n3, int kr1, int kr2, int kr3) {
-  const size_t nn = (size_t)kr1 * kr2 * kr3;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < nn; e += (size_t)gridDim.x * blockDim.x) {
-    const size_t yz = e / kr1;
-    const int y = (int)(yz % kr2), z = (int)(yz / kr2);
-    if (y >= n2 || z >= n3) v[e] = 0.0;
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -231,60 +232,77 @@ struct GParams {
   const double2* ph2;
   const double2* ph3;
   const int* sidx;           // (nhg) stick of each G
-  int nstick, L3;            // sticks; L3 = n3 + 1 positions m3 + h3 per stick
-  const double* sf;          // (nsp) blocks of (nstick x 2 L3): Re | Im of the structure factor
+  int nstick, lds, L3;       // sticks, their even leading dimension; L3 = n3 + 1 positions m3 + h3 per stick
+  const double* sf;          // (nsp) blocks of (lds x 2 L3): Re | Im of the structure factor
+  const double* gk;          // (3, nhg)
+  int nby;                   // stick operand of potfor: 2 blocks (X, X m3) or 3 (X G_k)
 };
 
-// eicalc + ppener: rho_e(G) = W(+G)/N, eivps, eirop, vtemp; block partials of
-// (eh, ei, ee, eps) over G != 0; the G = 0 terms are added on the host.  The
-// species structure factors sum_{a in sp} e^{-iG.R_a} come from the stick GEMM.
-__global__ __launch_bounds__(kThreads) void k_eicalc_ppener(GParams g, int n1, int n2, int n3,
-                                                            const double2* __restrict__ W, double scale,
-                                                            double2* __restrict__ rhog, double2* __restrict__ eirop,
-                                                            double2* __restrict__ eivps, double2* __restrict__ vtemp,
-                                                            double* __restrict__ part) {
+// eicalc + ppener, the scatter of vtemp and the stick operand of potfor in one
+// pass: rho_e(G) = W(+G)/N, eivps, eirop, V(+G) = vtemp, V(-G) = conj(vtemp)
+// (G = 0: vtemp; V zeroed before) and, with Y, for G != 0 on stick s at t = m3 +
+// h3 the rows b lds + s, columns 2t, 2t + 1 of Y = Re, Im of X_sp(G) (b = 0) and
+// X_sp(G) m3 (b = 1), or of X_sp(G) G_b (nby = 3), X_sp = rhops_sp scg
+// conj(rho_tot) + vps_sp conj(rho_e) (Y zeroed before).  Block partials of (eh,
+// ei, ee, eps) over G != 0; the values at G = 0 (rho_e, eirop, eivps) go to g0 for
+// the host.  The species structure factors sum_{a in sp} e^{-iG.R_a} come from
+// the stick GEMM.
+__global__ __launch_bounds__(kThreads) void k_eicalc_ppener(GParams g, const double2* __restrict__ W, double scale,
+                                                            double2* __restrict__ V, double* __restrict__ Y,
+                                                            double2* __restrict__ g0, double* __restrict__ part) {
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  const size_t ldy = (size_t)g.nby * g.lds, blk = ldy * 2 * g.L3;
   for (int ig = blockIdx.x * blockDim.x + threadIdx.x; ig < g.nhg; ig += gridDim.x * blockDim.x) {
-    const double2 w = W[g.gidx[2 * ig]];
+    const int ip = g.gidx[2 * ig], im = g.gidx[2 * ig + 1];
+    const double2 w = W[ip];
     const double2 re = make_double2(w.x * scale, w.y * scale);
     double2 ev = make_double2(0.0, 0.0), er = make_double2(0.0, 0.0);
-    const size_t ps = (size_t)(g.gm[3 * ig + 2] + g.h3) * g.nstick + g.sidx[ig];
+    const int m3 = g.gm[3 * ig + 2], st = g.sidx[ig];
+    const size_t ps = (size_t)(m3 + g.h3) * g.lds + st;
     for (int is = 0; is < g.nsp; ++is) {
-      const double* S = g.sf + (size_t)is * g.nstick * 2 * g.L3;
-      const double2 sf = make_double2(S[ps], S[ps + (size_t)g.L3 * g.nstick]);
+      const double* S = g.sf + (size_t)is * g.lds * 2 * g.L3;
+      const double2 sf = make_double2(S[ps], S[ps + (size_t)g.L3 * g.lds]);
       const double vp = g.vps[is + (size_t)g.nsp * ig], rp = g.rhops[is + (size_t)g.nsp * ig];
       ev.x += vp * sf.x; ev.y += vp * sf.y;
       er.x += rp * sf.x; er.y += rp * sf.y;
     }
-    rhog[ig] = re;
-    eirop[ig] = er;
-    eivps[ig] = ev;
     const double2 rt = make_double2(re.x + er.x, re.y + er.y);
     const double s = g.scg[ig];
     if (g.geq0 && ig == 0) {
-      vtemp[ig] = make_double2(s * rt.x, s * rt.y);
-    } else {
-      vtemp[ig] = make_double2(s * rt.x + ev.x, s * rt.y + ev.y);
-      acc[0] += s * (rt.x * rt.x + rt.y * rt.y);
-      acc[1] += s * (er.x * er.x + er.y * er.y);
-      acc[2] += s * (re.x * re.x + re.y * re.y);
-      acc[3] += re.x * ev.x + re.y * ev.y;          // Re(conj(rho_e) eivps)
+      V[ip] = make_double2(s * rt.x, s * rt.y);
+      g0[0] = re;
+      g0[1] = er;
+      g0[2] = ev;
+      continue;
+    }
+    const double2 vt = make_double2(s * rt.x + ev.x, s * rt.y + ev.y);
+    V[ip] = vt;
+    V[im] = make_double2(vt.x, -vt.y);
+    acc[0] += s * (rt.x * rt.x + rt.y * rt.y);
+    acc[1] += s * (er.x * er.x + er.y * er.y);
+    acc[2] += s * (re.x * re.x + re.y * re.y);
+    acc[3] += re.x * ev.x + re.y * ev.y;          // Re(conj(rho_e) eivps)
+    if (!Y) continue;
+    const double2 A = make_double2(s * rt.x, -s * rt.y);   // scg conj(rho_tot)
+    for (int is = 0; is < g.nsp; ++is) {
+      const double rp = g.rhops[is + (size_t)g.nsp * ig], vp = g.vps[is + (size_t)g.nsp * ig];
+      const double2 X = make_double2(rp * A.x + vp * re.x, rp * A.y - vp * re.y);
+      double* y = Y + is * blk + (size_t)(2 * (m3 + g.h3)) * ldy + st;
+      if (g.nby == 2) {
+        y[0] = X.x;
+        y[ldy] = X.y;
+        y[g.lds] = X.x * m3;
+        y[ldy + g.lds] = X.y * m3;
+      } else {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          y[(size_t)k * g.lds] = X.x * g.gk[3 * ig + k];
+          y[ldy + (size_t)k * g.lds] = X.y * g.gk[3 * ig + k];
+        }
+      }
     }
   }
   block_sum_store<4>(acc, part + 4 * (size_t)blockIdx.x, 4);
-}
-
-// W(+G) = vtemp, W(-G) = conj(vtemp) (G = 0: vtemp); W zeroed before
-__global__ void k_scatter_vtemp(GParams g, const double2* __restrict__ vtemp, double2* __restrict__ W) {
-  for (int ig = blockIdx.x * blockDim.x + threadIdx.x; ig < g.nhg; ig += gridDim.x * blockDim.x) {
-    const double2 v = vtemp[ig];
-    if (g.geq0 && ig == 0) {
-      W[g.gidx[0]] = v;
-    } else {
-      W[g.gidx[2 * ig]] = v;
-      W[g.gidx[2 * ig + 1]] = make_double2(v.x, -v.y);
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -292,39 +310,47 @@ __global__ void k_scatter_vtemp(GParams g, const double2* __restrict__ vtemp, do
 // z-sticks (m1, m2) of the density set.  With e^{-iG.R_a} = p1_a(m1) p2_a(m2)
 // p3_a(m3) (phase tables) and Q(s, a) = p1_a(m1_s) p2_a(m2_s):
 //   S_sp(s, m3) = sum_{a in sp} Q(s, a) p3_a(m3)                        (eicalc)
-//   T_k(s, a)   = sum_m3 p3_a(m3) X_sp(G) G_k,  G = (m1_s, m2_s, m3)     (potfor)
-//   F_k(a)      = -sum_s Im(Q(s, a) T_k(s, a))
+//   T_b(s, a)   = sum_m3 p3_a(m3) X_sp(G) m3^b,  G = (m1_s, m2_s, m3), b = 0, 1  (potfor)
+//   F_k(a)      = -sum_s Im(Q(s, a) (base_k(s) T_0(s, a) + b3_k T_1(s, a)))
+// since G_k = base_k(s) + m3 b3_k on a stick (checked against the G's that were
+// set; a set of which it does not hold takes three blocks X G_k instead).
 // Complex products run as real GEMMs: one operand holds (re, im) pairs along
 // the contraction index, the other the real 2 x 2 expansion of p3.
 // ---------------------------------------------------------------------------
 
-// Q (nstick x 2 nat, ld nstick): columns 2a, 2a + 1 = Re, Im of Q(s, a)
-__global__ void k_stick_q(const int* __restrict__ stk, int nstick, int n1, int n2, const double2* __restrict__ ph1,
-                          const double2* __restrict__ ph2, double* __restrict__ Q) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x, a = blockIdx.y;
-  if (s >= nstick) return;
-  const double2 p = cmul(ph1[(size_t)a * (n1 + 1) + stk[2 * s] + n1 / 2], ph2[(size_t)a * (n2 + 1) + stk[2 * s + 1] + n2 / 2]);
-  Q[(size_t)(2 * a) * nstick + s] = p.x;
-  Q[(size_t)(2 * a + 1) * nstick + s] = p.y;
-}
-
+// The operands of both products, in one launch (blockIdx.x < nqb: Q).
+// Q (lds x 2 nat): columns 2a, 2a + 1 = Re, Im of Q(s, a), zero on the padding row.
 // Bs (2 nat x 2 L3, ld 2 nat), S = Q Bs: rows 2a, 2a + 1 of column t (Re S)
 // hold (Re p3, -Im p3), of column L3 + t (Im S) (Im p3, Re p3).
 // Bf (2 L3 x 2 nat, ld 2 L3), T = Y Bf: per species a block of columns
 // [Re | Im] (atom a of a species with first atom a0 and na atoms: Re column
 // 2 a0 + (a - a0), Im column 2 a0 + na + (a - a0)); rows 2t, 2t + 1 hold
 // (Re p3, -Im p3) in the Re column and (Im p3, Re p3) in the Im column.
-__global__ void k_stick_p3(const double2* __restrict__ ph3, int nat, int n3, const int* __restrict__ sp_of,
-                           const int* __restrict__ sp_start, double* __restrict__ Bs, double* __restrict__ Bf) {
+__global__ void k_stick_ops(const int* __restrict__ stk, int nstick, int lds, int n1, int n2, int n3, int nat, int nqb,
+                            const double2* __restrict__ ph1, const double2* __restrict__ ph2,
+                            const double2* __restrict__ ph3, const int* __restrict__ sp_of,
+                            const int* __restrict__ sp_start, double* __restrict__ Q, double* __restrict__ Bs,
+                            double* __restrict__ Bf) {
+  const int a = blockIdx.y;
+  if ((int)blockIdx.x < nqb) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= lds) return;
+    double2 p = make_double2(0.0, 0.0);
+    if (s < nstick)
+      p = cmul(ph1[(size_t)a * (n1 + 1) + stk[2 * s] + n1 / 2], ph2[(size_t)a * (n2 + 1) + stk[2 * s + 1] + n2 / 2]);
+    Q[(size_t)(2 * a) * lds + s] = p.x;
+    Q[(size_t)(2 * a + 1) * lds + s] = p.y;
+    return;
+  }
   const int L3 = n3 + 1;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x, a = blockIdx.y;
+  const int t = (blockIdx.x - nqb) * blockDim.x + threadIdx.x;
   if (t >= L3) return;
   const double2 p = ph3[(size_t)a * L3 + t];
-  const size_t lds = 2 * (size_t)nat;
-  Bs[(size_t)t * lds + 2 * a] = p.x;
-  Bs[(size_t)t * lds + 2 * a + 1] = -p.y;
-  Bs[(size_t)(L3 + t) * lds + 2 * a] = p.y;
-  Bs[(size_t)(L3 + t) * lds + 2 * a + 1] = p.x;
+  const size_t ldb = 2 * (size_t)nat;
+  Bs[(size_t)t * ldb + 2 * a] = p.x;
+  Bs[(size_t)t * ldb + 2 * a + 1] = -p.y;
+  Bs[(size_t)(L3 + t) * ldb + 2 * a] = p.y;
+  Bs[(size_t)(L3 + t) * ldb + 2 * a + 1] = p.x;
   const int sp = sp_of[a], a0 = sp_start[sp], na = sp_start[sp + 1] - a0;
   const size_t ldf = 2 * (size_t)L3;
   double* re = Bf + (size_t)(2 * a0 + (a - a0)) * ldf;
@@ -335,54 +361,48 @@ __global__ void k_stick_p3(const double2* __restrict__ ph3, int nat, int n3, con
   im[2 * t + 1] = p.x;
 }
 
-// Y (nsp blocks of 3 nstick x 2 L3, ld 3 nstick, zeroed before): row
-// k nstick + s, columns 2t, 2t + 1 = Re, Im of X_sp(G) G_k for G != 0 on stick
-// s at t = m3 + h3, X_sp = rhops_sp scg conj(rho_tot) + vps_sp conj(rho_e)
-__global__ void k_stick_y(GParams g, const double* __restrict__ gk, const double2* __restrict__ rhog,
-                          const double2* __restrict__ eirop, double* __restrict__ Y) {
-  const size_t ldy = 3 * (size_t)g.nstick, blk = ldy * 2 * g.L3;
-  for (int ig = blockIdx.x * blockDim.x + threadIdx.x; ig < g.nhg; ig += gridDim.x * blockDim.x) {
-    if (g.geq0 && ig == 0) continue;
-    const int s = g.sidx[ig], t = g.gm[3 * ig + 2] + g.h3;
-    const double2 re = rhog[ig], er = eirop[ig];
-    const double sc = g.scg[ig];
-    const double2 A = make_double2(sc * (re.x + er.x), -sc * (re.y + er.y));   // scg conj(rho_tot)
-    const double2 B = make_double2(re.x, -re.y);                              // conj(rho_e)
-    const double gv[3] = {gk[3 * ig], gk[3 * ig + 1], gk[3 * ig + 2]};
-    for (int is = 0; is < g.nsp; ++is) {
-      const double rp = g.rhops[is + (size_t)g.nsp * ig], vp = g.vps[is + (size_t)g.nsp * ig];
-      const double2 X = make_double2(rp * A.x + vp * B.x, rp * A.y + vp * B.y);
-      double* y = Y + is * blk + s;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        y[(size_t)(2 * t) * ldy + (size_t)k * g.nstick] = X.x * gv[k];
-        y[(size_t)(2 * t + 1) * ldy + (size_t)k * g.nstick] = X.y * gv[k];
-      }
-    }
-  }
-}
-
-// fout[3a + k] = -scale sum_s Im(Q(s, a) T_k(s, a)); T (3 nstick x 2 nat, ld
-// 3 nstick) in the column order of Bf.  One workgroup per (a, k), fixed order.
+// fout[3 (c nat + a) + k] = -scale sum over the sticks of chunk c of Im(Q(s, a)
+// T(s, a)) with T_k = base_k(s) T_0 + b3_k T_1 (nby = 2; base (3, nstick)) or T_k
+// itself; T (nby lds x 2 nat) in the column order of Bf.  One workgroup per (a,
+// chunk), fixed order; the host adds the chunks.
+constexpr int kForceChunks = 4;
 __global__ __launch_bounds__(kThreads) void k_stick_force(const double* __restrict__ Q, const double* __restrict__ T,
-                                                          int nstick, const int* __restrict__ sp_of,
+                                                          int nstick, int lds, int nby,
+                                                          const double* __restrict__ base, double b0, double b1,
+                                                          double b2, const int* __restrict__ sp_of,
                                                           const int* __restrict__ sp_start, double scale,
                                                           double* __restrict__ fout) {
-  const int a = blockIdx.x, k = blockIdx.y;
+  const int a = blockIdx.x;
   const int sp = sp_of[a], a0 = sp_start[sp], na = sp_start[sp + 1] - a0;
-  const size_t ldt = 3 * (size_t)nstick;
-  const double* qr = Q + (size_t)(2 * a) * nstick;
-  const double* qi = qr + nstick;
-  const double* tr = T + (size_t)(2 * a0 + (a - a0)) * ldt + (size_t)k * nstick;
-  const double* ti = T + (size_t)(2 * a0 + na + (a - a0)) * ldt + (size_t)k * nstick;
-  double acc[1] = {0.0};
-  for (int s = threadIdx.x; s < nstick; s += kThreads) acc[0] += qr[s] * ti[s] + qi[s] * tr[s];
-  acc[0] *= -scale;
-  block_sum_store<1>(acc, fout + 3 * (size_t)a + k, 1);
+  const size_t ldt = (size_t)nby * lds;
+  const double* qr = Q + (size_t)(2 * a) * lds;
+  const double* qi = qr + lds;
+  const double* tr = T + (size_t)(2 * a0 + (a - a0)) * ldt;
+  const double* ti = T + (size_t)(2 * a0 + na + (a - a0)) * ldt;
+  const int per = (nstick + kForceChunks - 1) / kForceChunks;
+  const int s1 = min(nstick, ((int)blockIdx.y + 1) * per);
+  double acc[3] = {0.0, 0.0, 0.0};
+  for (int s = blockIdx.y * per + threadIdx.x; s < s1; s += kThreads) {
+    const double x = qr[s], y = qi[s];
+    if (nby == 2) {
+      const double t0 = x * ti[s] + y * tr[s], t1 = x * ti[s + lds] + y * tr[s + lds];
+      acc[0] += base[3 * s] * t0 + b0 * t1;
+      acc[1] += base[3 * s + 1] * t0 + b1 * t1;
+      acc[2] += base[3 * s + 2] * t0 + b2 * t1;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) acc[k] += x * ti[s + (size_t)k * lds] + y * tr[s + (size_t)k * lds];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) acc[k] *= -scale;
+  block_sum_store<3>(acc, fout + 3 * ((size_t)blockIdx.y * gridDim.x + a), 3);
 }
 
 // ---------------------------------------------------------------------------
-// Ewald real-space sum (rpiiint): block per atom l, threads over partners m;
+// Ewald real-space sum (rpiiint): blocks per atom l, threads over (image, partner m).
+// Bound by the FP64 arithmetic of erfc and exp (61 us at 256 atoms, 9 at 8; with a
+// block per atom and a thread per partner 93 and 74).
 // e_l = sum_m sum_images w zv_l zv_m erfc(r / rckj) / r with w = 1/2 (each
 // unordered pair is visited from both ends; the self images of l carry the
 // reference's 1/2), F_l = sum_{m != l} sum_images (erfc term + Gaussian term) r / r^2
@@ -401,7 +421,10 @@ __global__ __launch_bounds__(kThreads) void k_ewald(EParams p, double* __restric
   const int l = blockIdx.x;
   const int kl = p.sp_of[l];
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int m = threadIdx.x; m < p.nat; m += kThreads) {
+  const int ni = 2 * p.iesr + 1, nimg = ni * ni * ni;
+  for (int e = blockIdx.y * kThreads + threadIdx.x; e < p.nat * nimg; e += gridDim.y * kThreads) {
+    const int img = e / p.nat, m = e - img * p.nat;
+    const int ix = img / (ni * ni) - p.iesr, iy = img / ni % ni - p.iesr, iz = img % ni - p.iesr;
     const int km = p.sp_of[m];
     const double zv2 = p.zv[kl] * p.zv[km];
     if (fabs(zv2) < 1e-10) continue;
@@ -415,27 +438,23 @@ __global__ __launch_bounds__(kThreads) void k_ewald(EParams p, double* __restric
       for (int i = 0; i < 3; ++i) fr[i] -= nearbyint(fr[i]);
       for (int q = 0; q < 3; ++q) d[q] = fr[0] * p.a[q] + fr[1] * p.a[3 + q] + fr[2] * p.a[6 + q];
     }
-    for (int ix = -p.iesr; ix <= p.iesr; ++ix)
-      for (int iy = -p.iesr; iy <= p.iesr; ++iy)
-        for (int iz = -p.iesr; iz <= p.iesr; ++iz) {
-          if (tzero && ix == 0 && iy == 0 && iz == 0) continue;
-          double r[3];
-          for (int q = 0; q < 3; ++q) r[q] = d[q] + ix * p.a[q] + iy * p.a[3 + q] + iz * p.a[6 + q];
-          const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-          const double rl = sqrt(r2);
-          const double arg = rl / rckj;
-          if (arg > 20.0) continue;
-          const double add = zv2 * erfc(arg) / rl;
-          acc[0] += 0.5 * add;
-          if (!tzero) {
-            const double rep = (add + 2.0 * zv2 / sqrt(M_PI) * exp(-arg * arg) / rckj) / r2;
-            acc[1] += rep * r[0];
-            acc[2] += rep * r[1];
-            acc[3] += rep * r[2];
-          }
-        }
+    if (tzero && ix == 0 && iy == 0 && iz == 0) continue;
+    double r[3];
+    for (int q = 0; q < 3; ++q) r[q] = d[q] + ix * p.a[q] + iy * p.a[3 + q] + iz * p.a[6 + q];
+    const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+    const double rl = sqrt(r2);
+    const double arg = rl / rckj;
+    if (arg > 20.0) continue;
+    const double add = zv2 * erfc(arg) / rl;
+    acc[0] += 0.5 * add;
+    if (!tzero) {
+      const double rep = (add + 2.0 * zv2 / sqrt(M_PI) * exp(-arg * arg) / rckj) / r2;
+      acc[1] += rep * r[0];
+      acc[2] += rep * r[1];
+      acc[3] += rep * r[2];
+    }
   }
-  block_sum_store<4>(acc, out + 4 * (size_t)l, 4);
+  block_sum_store<4>(acc, out + 4 * ((size_t)blockIdx.y * p.nat + l), 4);
 }
 
 // projector structure factors on the wavefunction rows (device order):
@@ -462,56 +481,105 @@ void set_density_gset(mc_ctx* ctx, int nhg, const int* inyh, const double* hg, c
   auto& D = ctx->dens;
   MC_CHECK(nhg >= 1, MC_ERR_ARG, "set_density_gset: nhg < 1");
   const int nr[3] = {ctx->n1, ctx->n2, ctx->n3};
-  std::vector<int> gm((size_t)3 * nhg), gidx((size_t)2 * nhg);
-  std::vector<double> scg(nhg);
-  for (int ig = 0; ig < nhg; ++ig) {
-    int ip[3], im[3];
+  for (int ig = 0; ig < nhg; ++ig)
     for (int k = 0; k < 3; ++k) {
       const int m = inyh[3 * (size_t)ig + k] - (nr[k] / 2 + 1);
       MC_CHECK(m >= -nr[k] / 2 && m <= nr[k] / 2, MC_ERR_ARG, "set_density_gset: G index outside the mesh");
-      gm[3 * (size_t)ig + k] = m;
-      ip[k] = ((m % nr[k]) + nr[k]) % nr[k];
-      im[k] = ((-m % nr[k]) + nr[k]) % nr[k];
+      if (ig == 0 && ctx->geq0) MC_CHECK(m == 0, MC_ERR_ARG, "set_density_gset: first G must be G = 0");
     }
-    gidx[2 * (size_t)ig] = ip[0] + nr[0] * (ip[1] + nr[1] * ip[2]);
-    gidx[2 * (size_t)ig + 1] = im[0] + nr[0] * (im[1] + nr[1] * im[2]);
-    if (ig == 0 && ctx->geq0) {
-      MC_CHECK(gm[0] == 0 && gm[1] == 0 && gm[2] == 0, MC_ERR_ARG, "set_density_gset: first G must be G = 0");
-      scg[ig] = 0.0;
+  // device order: G = 0 first (geq0), then m1 fastest, m2, m3 (two stable counting
+  // sorts)
+  const int first = ctx->geq0 ? 1 : 0;
+  std::vector<int> perm(nhg), tmp(nhg);
+  for (int ig = 0; ig < nhg; ++ig) perm[ig] = ig;
+  const auto sort_by = [&](auto key, int nkey) {
+    std::vector<int> pos(nkey + 1, 0);
+    for (int j = first; j < nhg; ++j) ++pos[key(perm[j]) + 1];
+    for (int v = 0; v < nkey; ++v) pos[v + 1] += pos[v];
+    for (int j = first; j < nhg; ++j) tmp[first + pos[key(perm[j])]++] = perm[j];
+    perm.swap(tmp);
+    if (first) perm[0] = 0;
+  };
+  const int w1 = nr[0] + 2, w2 = nr[1] + 2;
+  sort_by([&](int ig) { return inyh[3 * (size_t)ig]; }, w1);
+  sort_by([&](int ig) { return inyh[3 * (size_t)ig + 1] + w2 * inyh[3 * (size_t)ig + 2]; }, w2 * (nr[2] + 2));
+  // z-sticks: the distinct (m1, m2) in the order (m2, m1), and the stick of each G
+  std::vector<int> sid((size_t)w1 * w2, -1);
+  for (int ig = 0; ig < nhg; ++ig) sid[inyh[3 * (size_t)ig] + (size_t)w1 * inyh[3 * (size_t)ig + 1]] = 0;
+  int nstick = 0;
+  std::vector<int> stk;
+  for (size_t e = 0; e < sid.size(); ++e)
+    if (sid[e] == 0) {
+      sid[e] = nstick++;
+      stk.push_back((int)(e % w1) - (nr[0] / 2 + 1));
+      stk.push_back((int)(e / w1) - (nr[1] / 2 + 1));
+    }
+  std::vector<int> gm((size_t)3 * nhg), gidx((size_t)2 * nhg), sidx(nhg);
+  std::vector<double> scg(nhg), gks((size_t)3 * nhg);
+  for (int j = 0; j < nhg; ++j) {
+    const size_t ig = perm[j];
+    int ip[3], im[3];
+    for (int k = 0; k < 3; ++k) {
+      const int m = inyh[3 * ig + k] - (nr[k] / 2 + 1);
+      gm[3 * (size_t)j + k] = m;
+      ip[k] = m < 0 ? m + nr[k] : m % nr[k];
+      im[k] = m > 0 ? nr[k] - m : -m % nr[k];
+      gks[3 * (size_t)j + k] = gk[3 * ig + k];
+    }
+    gidx[2 * (size_t)j] = ip[0] + nr[0] * (ip[1] + nr[1] * ip[2]);
+    gidx[2 * (size_t)j + 1] = im[0] + nr[0] * (im[1] + nr[1] * im[2]);
+    sidx[j] = sid[inyh[3 * ig] + (size_t)w1 * inyh[3 * ig + 1]];
+    if (j == 0 && ctx->geq0) {
+      scg[j] = 0.0;
     } else {
       MC_CHECK(hg[ig] > 0.0, MC_ERR_ARG, "set_density_gset: G = 0 after the first position");
-      scg[ig] = 4.0 * M_PI / (ctx->tpiba2 * hg[ig]);
+      scg[j] = 4.0 * M_PI / (ctx->tpiba2 * hg[ig]);
     }
   }
-  // z-sticks: the distinct (m1, m2) in increasing order and the stick of each G
-  const long long w2 = nr[1] + 1;
-  std::vector<long long> key(nhg);
-  for (int ig = 0; ig < nhg; ++ig)
-    key[ig] = (long long)(gm[3 * (size_t)ig] + nr[0] / 2) * w2 + (gm[3 * (size_t)ig + 1] + nr[1] / 2);
-  std::vector<long long> uk(key);
-  std::sort(uk.begin(), uk.end());
-  uk.erase(std::unique(uk.begin(), uk.end()), uk.end());
-  const int nstick = (int)uk.size();
-  std::vector<int> sidx(nhg), stk(2 * (size_t)nstick);
-  for (int ig = 0; ig < nhg; ++ig) sidx[ig] = (int)(std::lower_bound(uk.begin(), uk.end(), key[ig]) - uk.begin());
-  for (int st = 0; st < nstick; ++st) {
-    stk[2 * (size_t)st] = (int)(uk[st] / w2) - nr[0] / 2;
-    stk[2 * (size_t)st + 1] = (int)(uk[st] % w2) - nr[1] / 2;
+  // G_k = base_k(stick) + m3 b3_k: b3 from the stick with the widest range of m3,
+  // base from the first G of each stick; nby = 3 when the set does not fit that
+  std::vector<int> lo(nstick, -1), hi(nstick, -1);
+  for (int j = 0; j < nhg; ++j) {   // m3 rises with j behind G = 0
+    const int st = sidx[j];
+    if (lo[st] < 0 || gm[3 * (size_t)j + 2] < gm[3 * (size_t)lo[st] + 2]) lo[st] = j;
+    if (hi[st] < 0 || gm[3 * (size_t)j + 2] > gm[3 * (size_t)hi[st] + 2]) hi[st] = j;
   }
+  int wide = 0, span = -1;
+  for (int st = 0; st < nstick; ++st) {
+    const int d = gm[3 * (size_t)hi[st] + 2] - gm[3 * (size_t)lo[st] + 2];
+    if (d > span) {
+      span = d;
+      wide = st;
+    }
+  }
+  std::vector<double> base((size_t)3 * nstick);
+  double gmax = 0.0;
+  for (int k = 0; k < 3; ++k)
+    D.b3[k] = span > 0 ? (gks[3 * (size_t)hi[wide] + k] - gks[3 * (size_t)lo[wide] + k]) / span : 0.0;
+  for (int st = 0; st < nstick; ++st)
+    for (int k = 0; k < 3; ++k)
+      base[3 * (size_t)st + k] = gks[3 * (size_t)lo[st] + k] - gm[3 * (size_t)lo[st] + 2] * D.b3[k];
+  for (double x : gks) gmax = std::max(gmax, std::fabs(x));
+  D.nby = 2;
+  for (int j = 0; j < nhg && D.nby == 2; ++j)
+    for (int k = 0; k < 3; ++k)
+      if (!(std::fabs(base[3 * (size_t)sidx[j] + k] + gm[3 * (size_t)j + 2] * D.b3[k] - gks[3 * (size_t)j + k]) <=
+            1e-14 * gmax))
+        D.nby = 3;
   D.nstick = nstick;
-  D.d_sidx.ensure(sizeof(int) * sidx.size());
-  D.d_stk.ensure(sizeof(int) * stk.size());
-  MC_HIP(hipMemcpy(D.d_sidx.p, sidx.data(), sizeof(int) * sidx.size(), hipMemcpyHostToDevice));
-  MC_HIP(hipMemcpy(D.d_stk.p, stk.data(), sizeof(int) * stk.size(), hipMemcpyHostToDevice));
   D.nhg = nhg;
-  D.d_gm.ensure(sizeof(int) * gm.size());
-  D.d_gidx.ensure(sizeof(int) * gidx.size());
-  D.d_scg.ensure(sizeof(double) * nhg);
-  D.d_gk.ensure(sizeof(double) * 3 * (size_t)nhg);
-  MC_HIP(hipMemcpy(D.d_gm.p, gm.data(), sizeof(int) * gm.size(), hipMemcpyHostToDevice));
-  MC_HIP(hipMemcpy(D.d_gidx.p, gidx.data(), sizeof(int) * gidx.size(), hipMemcpyHostToDevice));
-  MC_HIP(hipMemcpy(D.d_scg.p, scg.data(), sizeof(double) * nhg, hipMemcpyHostToDevice));
-  MC_HIP(hipMemcpy(D.d_gk.p, gk, sizeof(double) * 3 * (size_t)nhg, hipMemcpyHostToDevice));
+  D.gperm = perm;
+  const auto put = [](DevBuf& b, const void* p, size_t bytes) {
+    b.ensure(bytes);
+    MC_HIP(hipMemcpy(b.p, p, bytes, hipMemcpyHostToDevice));
+  };
+  put(D.d_sidx, sidx.data(), sizeof(int) * sidx.size());
+  put(D.d_stk, stk.data(), sizeof(int) * stk.size());
+  put(D.d_base, base.data(), sizeof(double) * base.size());
+  put(D.d_gm, gm.data(), sizeof(int) * gm.size());
+  put(D.d_gidx, gidx.data(), sizeof(int) * gidx.size());
+  put(D.d_scg, scg.data(), sizeof(double) * scg.size());
+  put(D.d_gk, gks.data(), sizeof(double) * gks.size());
   D.ready = true;
   D.pp_ready = false;
 }
@@ -545,8 +613,14 @@ void set_local_pp(mc_ctx* ctx, int nsp, const int* na, const double* zv, const d
   MC_HIP(hipMemcpy(D.d_sp_of.p, sp_of.data(), sizeof(int) * sp_of.size(), hipMemcpyHostToDevice));
   MC_HIP(hipMemcpy(D.d_zv.p, zv, sizeof(double) * nsp, hipMemcpyHostToDevice));
   MC_HIP(hipMemcpy(D.d_raggio.p, raggio, sizeof(double) * nsp, hipMemcpyHostToDevice));
-  MC_HIP(hipMemcpy(D.d_vps.p, vps, sizeof(double) * (size_t)nsp * D.nhg, hipMemcpyHostToDevice));
-  MC_HIP(hipMemcpy(D.d_rhops.p, rhops, sizeof(double) * (size_t)nsp * D.nhg, hipMemcpyHostToDevice));
+  // in the device order of the G's
+  std::vector<double> x((size_t)nsp * D.nhg);
+  for (int w = 0; w < 2; ++w) {
+    const double* src = w ? rhops : vps;
+    for (int j = 0; j < D.nhg; ++j)
+      for (int is = 0; is < nsp; ++is) x[is + (size_t)nsp * j] = src[is + (size_t)nsp * D.gperm[j]];
+    MC_HIP(hipMemcpy((w ? D.d_rhops : D.d_vps).p, x.data(), sizeof(double) * x.size(), hipMemcpyHostToDevice));
+  }
   D.pp_ready = true;
   D.ions_ready = false;
 }
@@ -627,6 +701,9 @@ static GParams make_gparams(mc_ctx* ctx) {
   g.ph3 = D.d_ph3.as<double2>();
   g.sidx = D.d_sidx.as<int>();
   g.nstick = D.nstick;
+  g.lds = D.nstick + (D.nstick & 1);
+  g.gk = D.d_gk.as<double>();
+  g.nby = D.nby;
   g.L3 = ctx->n3 + 1;
   g.sf = nullptr;
   return g;
@@ -640,13 +717,11 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
   const GParams g = make_gparams(ctx);
   const size_t nw = (size_t)ctx->n1 * ctx->n2 * ctx->n3;
   const double nn = (double)nw;
+  // the mesh before and after the per-G pass
   D.w_W.ensure(sizeof(double2) * nw);
-  D.w_g.ensure(sizeof(double2) * 4 * (size_t)D.nhg);
+  D.w_V.ensure(sizeof(double2) * nw);
   double2* W = D.w_W.as<double2>();
-  double2* rhog = D.w_g.as<double2>();
-  double2* eirop = rhog + D.nhg;
-  double2* eivps = eirop + D.nhg;
-  double2* vtemp = eivps + D.nhg;
+  double2* V = D.w_V.as<double2>();
   const int tx = std::min(lines_for<double>(ctx->plan1), 16);
   // y / z passes keep lines at stride n + 1 in LDS: fit table + lines in kLdsBudget
   auto fit = [](int l, int n) { return std::max(1, std::min(l, (kLdsBudget / 16 - n) / (n + 1))); };
@@ -656,34 +731,47 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
   const size_t sh3 = sizeof(double2) * ((size_t)ctx->n3 + (size_t)(ctx->n3 + 1) * t3);
   const int gx_blocks = (ctx->n2 + tx - 1) / tx;
   const int n_xblk = gx_blocks * ctx->n3;
-  // partial-sum area: ppener (4 per block), xc (2 per x block), ion forces (3 per atom)
-  const size_t npart = 4 * (size_t)kRedBlocks + 2 * (size_t)n_xblk + 3 * (size_t)std::max(D.nat, 1);
-  D.w_part.ensure(sizeof(double) * npart);
+  // partial-sum area: ppener (4 per block), xc (2 per x block), the values at
+  // G = 0 (3 complex), ion forces (3 per atom and chunk)
+  const bool forces = fion_host && D.nat > 0;
+  const size_t nsum = 4 * (size_t)kRedBlocks + 2 * (size_t)n_xblk + 6;
+  const size_t nforce = forces ? 3 * (size_t)D.nat * kForceChunks : 0;
+  D.w_part.ensure(sizeof(double) * (nsum + 3 * (size_t)std::max(D.nat, 1) * kForceChunks));
   double* p_pp = D.w_part.as<double>();
   double* p_xc = p_pp + 4 * kRedBlocks;
-  double* f_out = p_xc + 2 * (size_t)n_xblk;
-  // stick operands: Q, the p3 expansions, the species structure factors
-  const int ns = D.nstick, L3 = ctx->n3 + 1, nat = D.nat;
-  const size_t sfblk = (size_t)ns * 2 * L3;
-  D.w_q.ensure(sizeof(double) * (size_t)ns * 2 * std::max(nat, 1));
+  double2* p_g0 = reinterpret_cast<double2*>(p_xc + 2 * (size_t)n_xblk);
+  double* f_out = p_pp + nsum;
+  // stick operands: Q, the p3 expansions, the species structure factors; for the
+  // forces Y and T
+  const int ns = D.nstick, ls = g.lds, L3 = ctx->n3 + 1, nat = D.nat, nby = D.nby;
+  const size_t sfblk = (size_t)ls * 2 * L3, yblk = nby * sfblk;
+  D.w_q.ensure(sizeof(double) * (size_t)ls * 2 * std::max(nat, 1));
   D.w_bs.ensure(sizeof(double) * 4 * (size_t)std::max(nat, 1) * L3);
   D.w_bf.ensure(sizeof(double) * 4 * (size_t)std::max(nat, 1) * L3);
   D.w_sf.ensure(sizeof(double) * sfblk * D.nsp);
   double* Q = D.w_q.as<double>();
   double* Sf = D.w_sf.as<double>();
+  double* Y = nullptr;
+  if (forces) {
+    D.w_y.ensure(sizeof(double) * yblk * D.nsp);
+    D.w_t.ensure(sizeof(double) * nby * (size_t)ls * 2 * nat);
+    Y = D.w_y.as<double>();
+    LAUNCH(MC_KID_VOFRHO, k_fill, dim3(1024), dim3(256), 0, Y, yblk * D.nsp, 0.0);
+  }
+  LAUNCH(MC_KID_VOFRHO, k_fill, dim3(1024), dim3(256), 0, (double*)V, 2 * nw, 0.0);
   if (nat > 0) {
-    LAUNCH(MC_KID_VOFRHO, k_stick_q, dim3((ns + 255) / 256, nat), dim3(256), 0, D.d_stk.as<int>(), ns, ctx->n1,
-           ctx->n2, g.ph1, g.ph2, Q);
-    LAUNCH(MC_KID_VOFRHO, k_stick_p3, dim3((L3 + 255) / 256, nat), dim3(256), 0, g.ph3, nat, ctx->n3,
-           D.d_sp_of.as<int>(), D.d_sp_start.as<int>(), D.w_bs.as<double>(), D.w_bf.as<double>());
+    const int nqb = (ls + 255) / 256;
+    LAUNCH(MC_KID_VOFRHO, k_stick_ops, dim3(nqb + (L3 + 255) / 256, nat), dim3(256), 0, D.d_stk.as<int>(), ns, ls,
+           ctx->n1, ctx->n2, ctx->n3, nat, nqb, g.ph1, g.ph2, g.ph3, D.d_sp_of.as<int>(), D.d_sp_start.as<int>(), Q,
+           D.w_bs.as<double>(), D.w_bf.as<double>());
   }
   {
     int a0 = 0;
     for (int is = 0; is < D.nsp; ++is) {
       const int na = D.na[is];
       if (na > 0)
-        gemm_nn_f64(ctx, Q + (size_t)2 * a0 * ns, ns, D.w_bs.as<double>() + 2 * a0, 2 * nat, ns, 2 * na, 2 * L3,
-                    1.0, 0.0, Sf + is * sfblk, ns, false, nullptr, MC_KID_VOFRHO);
+        gemm_nn_f64(ctx, Q + (size_t)2 * a0 * ls, ls, D.w_bs.as<double>() + 2 * a0, 2 * nat, ls, 2 * na, 2 * L3,
+                    1.0, 0.0, Sf + is * sfblk, ls, false, nullptr, MC_KID_VOFRHO);
       else
         LAUNCH(MC_KID_VOFRHO, k_fill, dim3(256), dim3(256), 0, Sf + is * sfblk, sfblk, 0.0);
       a0 += na;
@@ -706,57 +794,42 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
            dim3(kThreads), sh3, d, W, t3);
   });
   // per-G energies and potential
-  LAUNCH(MC_KID_VOFRHO, k_eicalc_ppener, dim3(kRedBlocks), dim3(kThreads), 0, gs, ctx->n1, ctx->n2, ctx->n3, W,
-         1.0 / nn, rhog, eirop, eivps, vtemp, p_pp);
-  if (fion_host && nat > 0) {
-    // potfor: Y = X G_k on the sticks, T = Y Bf per species, F = -Im sum_s Q T
-    const size_t yblk = 3 * sfblk;
-    D.w_y.ensure(sizeof(double) * yblk * D.nsp);
-    D.w_t.ensure(sizeof(double) * 3 * (size_t)ns * 2 * nat);
-    double* Y = D.w_y.as<double>();
+  LAUNCH(MC_KID_VOFRHO, k_eicalc_ppener, dim3(kRedBlocks), dim3(kThreads), 0, gs, W, 1.0 / nn, V, Y, p_g0, p_pp);
+  if (forces) {
+    // potfor: T = Y Bf per species, F = -Im sum_s Q T
     double* T = D.w_t.as<double>();
-    LAUNCH(MC_KID_VOFRHO, k_fill, dim3(1024), dim3(256), 0, Y, yblk * D.nsp, 0.0);
-    LAUNCH(MC_KID_VOFRHO, k_stick_y, dim3(kRedBlocks), dim3(256), 0, gs, D.d_gk.as<double>(), rhog, eirop, Y);
     int a0 = 0;
     for (int is = 0; is < D.nsp; ++is) {
       const int na = D.na[is];
       if (na > 0)
-        gemm_nn_f64(ctx, Y + is * yblk, 3 * ns, D.w_bf.as<double>() + (size_t)2 * a0 * 2 * L3, 2 * L3, 3 * ns,
-                    2 * L3, 2 * na, 1.0, 0.0, T + (size_t)2 * a0 * 3 * ns, 3 * ns, false, nullptr, MC_KID_VOFRHO);
+        gemm_nn_f64(ctx, Y + is * yblk, nby * ls, D.w_bf.as<double>() + (size_t)2 * a0 * 2 * L3, 2 * L3, nby * ls,
+                    2 * L3, 2 * na, 1.0, 0.0, T + (size_t)2 * a0 * nby * ls, nby * ls, false, nullptr,
+                    MC_KID_VOFRHO);
       a0 += na;
     }
-    LAUNCH(MC_KID_VOFRHO, k_stick_force, dim3(nat, 3), dim3(kThreads), 0, Q, T, ns, D.d_sp_of.as<int>(),
-           D.d_sp_start.as<int>(), 2.0 * ctx->omega * std::sqrt(ctx->tpiba2), f_out);
+    LAUNCH(MC_KID_VOFRHO, k_stick_force, dim3(nat, kForceChunks), dim3(kThreads), 0, Q, T, ns, ls, nby,
+           D.d_base.as<double>(), D.b3[0], D.b3[1], D.b3[2], D.d_sp_of.as<int>(), D.d_sp_start.as<int>(),
+           2.0 * ctx->omega * std::sqrt(ctx->tpiba2), f_out);
   }
-  LAUNCH(MC_KID_VOFRHO, k_fill, dim3(1024), dim3(256), 0, (double*)W, 2 * nw, 0.0);
-  LAUNCH(MC_KID_VOFRHO, k_scatter_vtemp, dim3(kRedBlocks), dim3(kThreads), 0, g, vtemp, W);
   with_length(ctx->n3, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dyz<decltype(NN)::value, 1, 3>), dim3((ctx->n1 + t3 - 1) / t3, ctx->n2),
-           dim3(kThreads), sh3, d, W, t3);
+           dim3(kThreads), sh3, d, V, t3);
   });
   with_length(ctx->n2, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dyz<decltype(NN)::value, 1, 2>), dim3((ctx->n1 + t2 - 1) / t2, ctx->n3),
-           dim3(kThreads), sh2, d, W, t2);
+           dim3(kThreads), sh2, d, V, t2);
   });
   with_length(ctx->n1, [&](auto NN) {
     LAUNCH(MC_KID_VOFRHO, (k_dx_inv_xc<decltype(NN)::value>), dim3(gx_blocks, ctx->n3), dim3(kThreads), shx, d,
-           W, rho, v, tx, p_xc);
+           V, rho, v, tx, p_xc);
   });
-  if (ctx->kr2 > ctx->n2 || ctx->kr3 > ctx->n3)
-    LAUNCH(MC_KID_VOFRHO, k_pad_zero, dim3(1024), dim3(256), 0, v, ctx->n2, ctx->n3, ctx->kr1, ctx->kr2, ctx->kr3);
   // host: fixed-order sums of the partials and the G = 0 terms
-  std::vector<double> hp(4 * (size_t)kRedBlocks + 2 * (size_t)n_xblk);
+  // (one read-back: the force chunks follow the sums)
+  std::vector<double> hp(nsum + nforce);
   dl_add(ctx, hp.data(), p_pp, sizeof(double) * hp.size());
-  std::vector<double> hf(3 * (size_t)D.nat);
-  if (fion_host && D.nat > 0)
-    dl_add(ctx, hf.data(), f_out, sizeof(double) * hf.size());
-  double2 g0[3] = {};
-  if (ctx->geq0) {
-    dl_add(ctx, &g0[0], rhog, sizeof(double2));
-    dl_add(ctx, &g0[1], eirop, sizeof(double2));
-    dl_add(ctx, &g0[2], eivps, sizeof(double2));
-  }
   dl_finish(ctx);
+  const double* hf = hp.data() + nsum;
+  const double* g0 = hp.data() + nsum - 6;   // rho_e, eirop, eivps at G = 0 (re, im)
   double s[4] = {0, 0, 0, 0};
   for (int b = 0; b < kRedBlocks; ++b)
     for (int q = 0; q < 4; ++q) s[q] += hp[4 * (size_t)b + q];
@@ -768,8 +841,8 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
   double vploc = 0.0;
   if (ctx->geq0) {
     // scg(G=0) = 0: only the local pseudopotential term survives at G = 0
-    vploc = g0[2].x;
-    s[3] += 0.5 * (g0[2].x * g0[0].x + g0[2].y * g0[0].y);
+    vploc = g0[4];
+    s[3] += 0.5 * (g0[4] * g0[0] + g0[5] * g0[1]);
   }
   if (energies) {
     energies[0] = s[0] * ctx->omega;         // ehep
@@ -780,8 +853,8 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
     energies[5] = sxc * ctx->omega / nn;     // exc
     energies[6] = vsum * ctx->omega / nn;    // vxc
   }
-  if (fion_host)
-    for (size_t e = 0; e < hf.size(); ++e) fion_host[e] += hf[e];
+  for (size_t e = 0; e < (forces ? 3 * (size_t)nat : 0); ++e)
+    for (int c = 0; c < kForceChunks; ++c) fion_host[e] += hf[(size_t)c * 3 * nat + e];
 }
 
 void ewald(mc_ctx* ctx, int iesr, double* esr, double* eself, double* fion_host) {
@@ -807,16 +880,20 @@ void ewald(mc_ctx* ctx, int iesr, double* esr, double* eself, double* fion_host)
   p.sp_of = D.d_sp_of.as<int>();
   p.zv = D.d_zv.as<double>();
   p.raggio = D.d_raggio.as<double>();
-  D.w_part.ensure(sizeof(double) * 4 * (size_t)nat);
-  LAUNCH(MC_KID_VOFRHO, k_ewald, dim3(nat), dim3(kThreads), 0, p, D.w_part.as<double>());
-  std::vector<double> h(4 * (size_t)nat);
+  // workgroups per atom: enough for the chip, each with several passes of its threads
+  const long long pairs = (long long)nat * (2 * iesr + 1) * (2 * iesr + 1) * (2 * iesr + 1);
+  const int ny = (int)std::max(1LL, std::min<long long>((2048 + nat - 1) / nat, pairs / (2 * kThreads)));
+  D.w_part.ensure(sizeof(double) * 4 * (size_t)nat * ny);
+  LAUNCH(MC_KID_VOFRHO, k_ewald, dim3(nat, ny), dim3(kThreads), 0, p, D.w_part.as<double>());
+  std::vector<double> h(4 * (size_t)nat * ny);
   dl_add(ctx, h.data(), D.w_part.p, sizeof(double) * h.size());
   dl_finish(ctx);
   double e = 0.0;
-  for (int l = 0; l < nat; ++l) {
-    e += h[4 * (size_t)l];
+  for (size_t b = 0; b < h.size() / 4; ++b) {
+    const size_t l = b % nat;
+    e += h[4 * b];
     if (fion_host)
-      for (int q = 0; q < 3; ++q) fion_host[3 * (size_t)l + q] += h[4 * (size_t)l + 1 + q];
+      for (int q = 0; q < 3; ++q) fion_host[3 * l + q] += h[4 * b + 1 + q];
   }
   if (esr) *esr = e;
 }

@@ -109,3 +109,27 @@ def test_vofrho_requires_setup(gpu):
     with pytest.raises(_lib.McError):
         ctx.nat_ions = 3
         ctx.vofrho(np.zeros(int(np.prod(sysm.cell.kr))))
+
+
+@pytest.mark.parametrize("affine", [True, False])
+@pytest.mark.parametrize("a, ecut", [(9.0, 25.0), (11.0, 30.0)])
+def test_vofrho_g_order(gpu, affine, a, ecut):
+    """The caller's order of the G's does not matter behind G = 0, and G vectors
+    that are no affine function of the index along a z-stick take the three
+    potfor blocks X G_k (bounds of test_vofrho_parity)."""
+    sysm, ctx, L, rho, inyh, gk, zv, rg, vps, rhops, frac = _case(a, 5, ecut, 6, seed=11)
+    hg = sysm.gset.hg
+    rng = np.random.default_rng(2)
+    if not affine:
+        gk = gk * (1.0 + 0.1 * rng.random(gk.shape))
+    p = np.concatenate([[0], 1 + rng.permutation(hg.size - 1)])
+    ctx.set_density_gset(inyh[p], hg[p], gk[p])
+    ctx.set_local_pp([5], zv, rg, np.asfortranarray(vps[:, p]), np.asfortranarray(rhops[:, p]))
+    ctx.set_ions(sysm.tau, sysm.cell.avec)
+    v, en, f = ctx.vofrho(rho)
+    ov, oen, of, _ = oracle.vofrho(L, inyh, hg, gk, [5], vps, rhops, frac, rho)
+    assert rel(v, ov) < 1e-12
+    for k in ("ehep", "ehii", "ehee", "epseu", "exc", "vxc"):
+        assert en[k] == pytest.approx(oen[k], rel=1e-11), k
+    assert en["vploc"] == pytest.approx(oen["vploc"], rel=1e-12, abs=1e-15)
+    assert rel(f, of) < 1e-10
