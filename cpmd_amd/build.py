@@ -17,7 +17,7 @@ CSRC = PKG / "csrc"
 LIB = PKG / "libmicpmd.so"
 
 HIP_SOURCES = ["context.hip", "wfft.hip", *(f"wfft_len_{i}.hip" for i in range(1, 8)), "gemm.hip",
-               "gemm_f64.hip", "gemm_x3.hip", "gemm_planes.hip", "ortho.hip", "chol.hip", "vofrho.hip",
+               "gemm_f64.hip", "gemm_x3.hip", "gemm_planes.hip", "ortho.hip", "chol.hip", "invsqrt.hip", "vofrho.hip",
                "capi.hip", "restart.hip", "probe.hip"]
 
 HIPCC_FLAGS = [

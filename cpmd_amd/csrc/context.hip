@@ -901,6 +901,7 @@ int mc_ctx_destroy(mc_ctx* ctx) {
   for (auto e : ctx->timer.pool) (void)hipEventDestroy(e);
   if (ctx->h_stage_done) (void)hipEventDestroy(ctx->h_stage_done);
   if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
+  if (ctx->h_down_done) (void)hipEventDestroy(ctx->h_down_done);
   if (ctx->h_down) (void)hipHostFree(ctx->h_down);
   if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;

@@ -278,6 +278,7 @@ struct mc_ctx {
     size_t off, bytes;
   };
   std::vector<DlCopy> h_down_pending;
+  hipEvent_t h_down_done = nullptr;   // a result copied while more work is queued (invsqrt.hip)
 
   // stick layout (see context.hip for the definitions)
   int n_own = 0;        // owner sticks (hold half-sphere G's); owner 0 is (0,0)
@@ -501,6 +502,9 @@ void gemm_tn_x3(mc_ctx* ctx, const double* A, int lda, const double* B, int ldb,
                 bool g0corr, bool symmetric, double* out, int ldo, const ProjA* proj);
 void gemm_nn_x3(mc_ctx* ctx, const double* A, int lda, const double* G, int ldgm, int M, int k, int n, double alpha,
                 double beta, double* D, int ldd, bool upper_g, const FnlEpi* epi);
+
+// Zout = S^-1/2 (n x n, symmetric positive definite; invsqrt.hip)
+void inv_sqrt(mc_ctx* ctx, const double* S, int n, double* Zout, int* iters);
 
 // orthonormalisation and projectors (ortho.hip)
 void ovlap_dev(mc_ctx* ctx, int n, double* a_dev, int lda, const double2* c1, const double2* c2);

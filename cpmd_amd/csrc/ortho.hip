@@ -286,57 +286,6 @@ void rgs_dev(mc_ctx* ctx, double2* c, int n, double* smat_host) {
   }
 }
 
-// Z = S^{-1/2} by the coupled Newton-Schulz iteration on S/c, c = ||S||_F:
-// T = (3I - Z Y)/2, Y <- Y T, Z <- T Z; Y -> (S/c)^{1/2}, Z -> (S/c)^{-1/2}.
-static void inv_sqrt(mc_ctx* ctx, const double* S, int n, double* Zout, int* iters) {
-  double* Y = small(ctx, 2, n);
-  double* Z = small(ctx, 3, n);
-  double* T = small(ctx, 4, n);
-  double* W = small(ctx, 5, n);
-  std::vector<double> hs((size_t)n * n);
-  MC_HIP(hipMemcpyAsync(hs.data(), S, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-  MC_HIP(hipStreamSynchronize(ctx->stream));
-  double fro = 0.0;
-  for (double v : hs) fro += v * v;
-  fro = std::sqrt(fro);
-  MC_CHECK(fro > 0.0 && std::isfinite(fro), MC_ERR_ARG, "lowdin: zero or non-finite overlap matrix");
-  // scale so that ||I - S/c||_2 < 1 when S is close to I: use c = max(1, ||S||_2 bound)
-  double cmax = 0.0;
-  for (int j = 0; j < n; ++j) {
-    double r = 0.0;
-    for (int i = 0; i < n; ++i) r += std::fabs(hs[i + (size_t)n * j]);
-    cmax = std::max(cmax, r);
-  }
-  const double c = cmax > 1.0 ? cmax : 1.0;   // ||S||_2 <= ||S||_1 (symmetric)
-  dim3 g2((n + 255) / 256, n);
-  hipLaunchKernelGGL(k_axpby_eye, g2, dim3(256), 0, ctx->stream, S, 1.0 / c, 0.0, (const double*)nullptr, 0.0, Y, n);
-  hipLaunchKernelGGL(k_axpby_eye, g2, dim3(256), 0, ctx->stream, S, 0.0, 1.0, (const double*)nullptr, 0.0, Z, n);
-  MC_HIP(hipGetLastError());
-  int it = 0;
-  const int maxit = 100;
-  bool done = false;
-  for (it = 1; it <= maxit; ++it) {
-    gemm_nn(ctx, Z, n, Y, n, n, n, n, 1.0, 0.0, W, n, false, nullptr);                 // W = Z Y
-    hipLaunchKernelGGL(k_axpby_eye, g2, dim3(256), 0, ctx->stream, W, -0.5, 1.5, (const double*)nullptr, 0.0, T, n);
-    MC_HIP(hipGetLastError());
-    gemm_nn(ctx, Y, n, T, n, n, n, n, 1.0, 0.0, W, n, false, nullptr);                 // W = Y T
-    MC_HIP(hipMemcpyAsync(Y, W, sizeof(double) * n * n, hipMemcpyDeviceToDevice, ctx->stream));
-    gemm_nn(ctx, T, n, Z, n, n, n, n, 1.0, 0.0, W, n, false, nullptr);                 // W = T Z
-    MC_HIP(hipMemcpyAsync(Z, W, sizeof(double) * n * n, hipMemcpyDeviceToDevice, ctx->stream));
-    if (done) break;
-    // ||T - I||: converged once the correction is at rounding level; one more sweep then
-    hipLaunchKernelGGL(k_axpby_eye, g2, dim3(256), 0, ctx->stream, T, 1.0, -1.0, (const double*)nullptr, 0.0, W, n);
-    const double dev = max_abs_diff(ctx, W, nullptr, (size_t)n * n);
-    MC_CHECK(std::isfinite(dev), MC_ERR_NOCONV, "lowdin: Newton-Schulz iteration diverged");
-    if (dev < 1e-15 * n) done = true;
-  }
-  MC_CHECK(done, MC_ERR_NOCONV, "lowdin: Newton-Schulz iteration did not converge in 100 steps");
-  hipLaunchKernelGGL(k_axpby_eye, g2, dim3(256), 0, ctx->stream, Z, 1.0 / std::sqrt(c), 0.0, (const double*)nullptr,
-                     0.0, Zout, n);
-  MC_HIP(hipGetLastError());
-  if (iters) *iters = it;
-}
-
 void lowdin_dev(mc_ctx* ctx, double2* c, int n, int* iters) {
   if (n <= 0) return;
   MC_CHECK(n < kX3Min, MC_ERR_UNSUPPORTED, "lowdin: nstate beyond 16383");
