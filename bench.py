@@ -501,7 +501,7 @@ def main():
 
     def tn_kernel_roofline():
         """The A^T B contraction kernel (k_tn_planes in the split-bf16 paths,
-        k_gemm_tn in FP64): the algorithm's MFMA flops per step (6 bf16
+        k_tn_f64 in FP64): the algorithm's MFMA flops per step (6 bf16
         products per FP64-equivalent product for the 3-part split, symmetric
         overlaps counted once) over its time per step."""
         split = head in ("mixed", "bf16x3")
