@@ -36,7 +36,7 @@ __device__ __forceinline__ double lane_value(double v, int src) {
 // rows: one wave (lane = column) eliminates within the panel in registers, the
 // pivot row's entries taken lane by lane, and all waves update the rows behind
 // it.  The panel loop stays rolled: fully unrolled, the instructions alone took
-// 180 us to fetch (this @@).  A pivot that is not positive ends the
+// 180 us to fetch (this one: 46).  A pivot that is not positive ends the
 // factorisation: *info = its order.
 __device__ void factor_block(double* T, double* Y, double* inv, int nb, int kb, double* __restrict__ S, int lds,
                              double* __restrict__ X, int ldx, int* info, int* bad) {
