@@ -3,22 +3,23 @@
 //
 //   Y_0 = S/c, Z_0 = I;  T = 3/2 I - 1/2 Z Y,  Y <- Y T,  Z <- T Z;  Z -> sqrt(c) S^-1/2
 //
-// All of these are polynomials in S, hence symmetric: a product A B is formed as
-// A^T B from contiguous columns, for the tiles on and above the diagonal only, and
-// stored to both triangles, which keeps the iterates symmetric to the last bit.
+// The iterates commute and are symmetric only up to rounding, and the iteration is
+// stable only while its products are those of the factors as they are, in this order:
+// formed as A^T B, or from the tiles above the diagonal mirrored below it, they
+// amplify the commutator, and S of a condition of 1e2 or 1e3 diverges (with true
+// products it converges to 1e6 and beyond).  So every tile is formed, A read by its rows.
 //
 // At a few hundred states a product is bound by latency, not by the matrix cores
-// (512: 0.27 GF, 4 us at 68 TF/s): it has to be cut into enough workgroups.
-// k_sym_product takes 32 x 32 tiles (136 at 512), the K range split over the four
-// waves of a workgroup and added in LDS, operands straight from L2 into registers
-// one group of 32 k ahead.  Its epilogue forms T and the largest |T - I|, and the
-// products Y T and T Z share a launch, so that an iteration is two launches
-// (17 and 18 us at 512 states; as three general products of 36 us with 64 workgroups,
-// two copies, two element passes, a reduction and a wait of the host it took 160).
-// lowdin of 67 states: 0.43 -> 0.15 ms; 512 / 1024 / 4096 states over 12,443 / 17,133 plane
-// waves 2.2 / 6.6 / 152 -> 0.9 / 3.4 / 93 ms.  The host reads
-// max |T - I| while the next iteration runs, which is needed in any case: one more
-// follows the one that has converged.
+// (512: 0.27 GF, 4 us at 68 TF/s): it has to be cut into enough workgroups.  k_product
+// takes 32 x 32 tiles (256 at 512), the K range split over the four waves of a
+// workgroup and added in LDS, operands straight from L2 into registers one group of 32
+// k ahead.  Its epilogue forms T and the largest |T - I|, and the products Y T and T Z
+// share a launch, so that an iteration is two launches (as three general products of 36
+// us with 64 workgroups, two copies, two element passes, a reduction and a wait of the
+// host it took 160 us at 512 states).  lowdin of 67 states: 0.53 -> 0.17 ms; 512 / 1024 /
+// 4096 states over 12,443 / 17,133 plane waves 2.2 / 6.6 / 151 -> 0.9 / 3.7 / 114 ms.  The
+// host reads max |T - I| while the next iteration runs, which is needed in any case: one
+// more follows the one that has converged.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -82,41 +83,38 @@ __global__ void k_finish(const double* __restrict__ Z, int n, int ld, double s, 
   if (i < n) out[i + (size_t)j * n] = s * Z[i + (size_t)j * ld];
 }
 
-struct SymProduct {
+struct Product {
   const double* a;
   const double* b;
   double* d;
 };
 
-// d = alpha a b + beta I (n x n, ld a multiple of kPad, zero behind n) for
-// symmetric a, b that commute; blockIdx.x = tile on or above the diagonal,
-// blockIdx.y = product.  dev (may be null): the bits of max |d - I|, which order
+// d = alpha a b + beta I (n x n, ld a multiple of kPad, zero behind n); blockIdx.x =
+// tile, blockIdx.y = product.  dev (may be null): the bits of max |d - I|, which order
 // like the values, with NaN above all.
-__global__ __launch_bounds__(256) void k_sym_product(SymProduct p0, SymProduct p1, int n, int ld, double alpha,
-                                                     double beta, unsigned long long* __restrict__ dev) {
+__global__ __launch_bounds__(256) void k_product(Product p0, Product p1, int n, int ld, int nt, double alpha,
+                                                 double beta, unsigned long long* __restrict__ dev) {
   __shared__ double part[4][32 * 33];
-  const SymProduct p = blockIdx.y ? p1 : p0;
-  int tj = (int)((sqrtf(8.0f * blockIdx.x + 1.0f) - 1.0f) * 0.5f);
-  while ((tj + 1) * (tj + 2) / 2 <= (int)blockIdx.x) ++tj;
-  while (tj * (tj + 1) / 2 > (int)blockIdx.x) --tj;
-  const int ti = blockIdx.x - tj * (tj + 1) / 2;
-  const int i0 = 32 * ti, j0 = 32 * tj;
+  const Product p = blockIdx.y ? p1 : p0;
+  const int i0 = 32 * ((int)blockIdx.x % nt), j0 = 32 * ((int)blockIdx.x / nt);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lq = lane >> 4;
   const int per = ld / 4, k0 = wave * per;
-  const double* pa = p.a + (size_t)(i0 + li) * ld + k0 + 2 * lq;   // columns i0 + li, + 16
+  // a by rows: a lane holds the rows 2 li, 2 li + 1 of one k (a column's 32 rows are 256
+  // contiguous bytes); b by columns j0 + li, + 16, two k at a time
+  const double* pa = p.a + i0 + 2 * li + (size_t)(k0 + 2 * lq) * ld;
   const double* pb = p.b + (size_t)(j0 + li) * ld + k0 + 2 * lq;
   const size_t c16 = (size_t)16 * ld;
-  d2 f[2][4][4];   // [stage][step of 8 k][a0, a1, b0, b1]
+  d2 f[2][4][4];   // [stage][step of 8 k][a at k = 2 lq, 2 lq + 1, b0, b1]
   const auto load = [&](int k, int st) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      f[st][u][0] = *reinterpret_cast<const d2*>(pa + k + 8 * u);
-      f[st][u][1] = *reinterpret_cast<const d2*>(pa + c16 + k + 8 * u);
+      f[st][u][0] = *reinterpret_cast<const d2*>(pa + (size_t)(k + 8 * u) * ld);
+      f[st][u][1] = *reinterpret_cast<const d2*>(pa + (size_t)(k + 8 * u + 1) * ld);
       f[st][u][2] = *reinterpret_cast<const d2*>(pb + k + 8 * u);
       f[st][u][3] = *reinterpret_cast<const d2*>(pb + c16 + k + 8 * u);
     }
   };
-  d4 acc[2][2];
+  d4 acc[2][2];   // [row of the pair][column block]
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -130,7 +128,7 @@ __global__ __launch_bounds__(256) void k_sym_product(SymProduct p0, SymProduct p
         for (int a = 0; a < 2; ++a)
 #pragma unroll
           for (int b = 0; b < 2; ++b)
-            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(s ? f[st][u][a].y : f[st][u][a].x,
+            acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a ? f[st][u][s].y : f[st][u][s].x,
                                                              s ? f[st][u][2 + b].y : f[st][u][2 + b].x, acc[a][b], 0, 0, 0);
   };
   load(0, 0);
@@ -147,25 +145,20 @@ __global__ __launch_bounds__(256) void k_sym_product(SymProduct p0, SymProduct p
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) part[wave][(16 * b + li) * 33 + 16 * a + 4 * r + lq] = acc[a][b][r];
+      for (int r = 0; r < 4; ++r) part[wave][(16 * b + li) * 33 + 2 * (4 * r + lq) + a] = acc[a][b][r];
   __syncthreads();
   double big = 0.0;
   bool bad = false;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int x = threadIdx.x & 31, y = (threadIdx.x >> 5) + 8 * q;
-    const auto value = [&](int i, int j) {   // tile entry; on a diagonal tile the upper one of both
-      const int e = ti == tj ? max(i, j) * 33 + min(i, j) : j * 33 + i;
-      return alpha * ((part[0][e] + part[1][e]) + (part[2][e] + part[3][e])) + (i0 + i == j0 + j ? beta : 0.0);
-    };
-    if (i0 + x < n && j0 + y < n) {
-      const double v = value(x, y);
-      p.d[i0 + x + (size_t)(j0 + y) * ld] = v;
-      const double t = fabs(v - (i0 + x == j0 + y ? 1.0 : 0.0));
-      bad |= !(t <= big) && !(t > big);
-      big = fmax(big, t);
-    }
-    if (ti != tj && j0 + x < n && i0 + y < n) p.d[j0 + x + (size_t)(i0 + y) * ld] = value(y, x);
+    const int x = threadIdx.x & 31, y = (threadIdx.x >> 5) + 8 * q, e = y * 33 + x;
+    if (i0 + x >= n || j0 + y >= n) continue;
+    const double one = i0 + x == j0 + y ? 1.0 : 0.0;
+    const double v = alpha * ((part[0][e] + part[1][e]) + (part[2][e] + part[3][e])) + one * beta;
+    p.d[i0 + x + (size_t)(j0 + y) * ld] = v;
+    const double t = fabs(v - one);
+    bad |= t != t;
+    big = fmax(big, t);
   }
   if (!dev) return;
   if (bad) big = __longlong_as_double(0x7ff8000000000000LL);
@@ -220,12 +213,11 @@ void inv_sqrt(mc_ctx* ctx, const double* S, int n, double* Zout, int* iters) {
   hipLaunchKernelGGL(k_start, dim3((unsigned)std::min<size_t>(1024, (nn + 255) / 256)), dim3(256), 0, ctx->stream, S, n,
                      ld, 1.0 / c, Y[0], Z[0], Y[1], dev, maxit + 1);
   MC_HIP(hipGetLastError());
-  const dim3 one(nt * (nt + 1) / 2), two(nt * (nt + 1) / 2, 2);
   const auto sweep = [&](int it) {   // iterate it from the buffers (it - 1) % 2
     const int o = (it - 1) & 1, w = it & 1;
-    const SymProduct zy = {Z[o], Y[o], T}, yt = {Y[o], T, Y[w]}, tz = {T, Z[o], Z[w]};
-    hipLaunchKernelGGL(k_sym_product, one, dim3(256), 0, ctx->stream, zy, zy, n, ld, -0.5, 1.5, dev + it);
-    hipLaunchKernelGGL(k_sym_product, two, dim3(256), 0, ctx->stream, yt, tz, n, ld, 1.0, 0.0,
+    const Product zy = {Z[o], Y[o], T}, yt = {Y[o], T, Y[w]}, tz = {T, Z[o], Z[w]};
+    hipLaunchKernelGGL(k_product, dim3(nt * nt), dim3(256), 0, ctx->stream, zy, zy, n, ld, nt, -0.5, 1.5, dev + it);
+    hipLaunchKernelGGL(k_product, dim3(nt * nt, 2), dim3(256), 0, ctx->stream, yt, tz, n, ld, nt, 1.0, 0.0,
                        (unsigned long long*)nullptr);
     MC_HIP(hipGetLastError());
   };
