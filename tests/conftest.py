@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 from pathlib import Path
@@ -28,3 +29,13 @@ def gpu():
     if not gpu_available():
         pytest.fail("GPU test selected but no GPU / libmicpmd.so available")
     return True
+
+
+@pytest.fixture(autouse=True)
+def _no_leftovers(request):
+    """A caught exception that a test keeps in a local holds the test's frame in a
+    reference cycle, and with it the contexts and device arrays there.  They are
+    freed before a GPU test begins, not when the collector happens to run: tests
+    that read the device memory in use would see it fall."""
+    if request.node.get_closest_marker("gpu"):
+        gc.collect()
