@@ -400,15 +400,20 @@ __global__ __launch_bounds__(kThreads) void k_stick_force(const double* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Ewald real-space sum (rpiiint): blocks per atom l, threads over (image, partner m).
-// Bound by the FP64 arithmetic of erfc and exp (61 us at 256 atoms, 9 at 8; with a
-// block per atom and a thread per partner 93 and 74).
+// Ewald real-space sum (rpiiint): blocks per atom l, threads over (partner m, share
+// of the images); the vector to m is reduced to the cell once per thread.  Bound by
+// FP64 arithmetic: erfc and exp where most images lie inside the cut-off, the
+// distance to the image where they do not.  The whole call with two images per
+// direction: 8 atoms 19 us, 256 45, 4096 2.85 ms; with one thread per partner at every
+// size 85, 49 and 2.85 (dealing single (image, partner) pairs, the vector formed anew
+// for each: 21, 88 and 11.1).
 // e_l = sum_m sum_images w zv_l zv_m erfc(r / rckj) / r with w = 1/2 (each
 // unordered pair is visited from both ends; the self images of l carry the
 // reference's 1/2), F_l = sum_{m != l} sum_images (erfc term + Gaussian term) r / r^2
 // ---------------------------------------------------------------------------
 struct EParams {
   int nat, iesr;
+  int ncol, nz;     // shares of a partner's images: of the (ix, iy), and of the iz
   double a[9];      // a[3 i + q]: component q of lattice vector i
   double inv[9];    // inv[3 q + i]: fractional coordinate i of a Cartesian vector
   const double* tau;
@@ -417,14 +422,22 @@ struct EParams {
   const double* raggio;
 };
 
-__global__ __launch_bounds__(kThreads) void k_ewald(EParams p, double* __restrict__ out) {
+template <bool SHARES>
+__global__ __launch_bounds__(kThreads, 4) void k_ewald(EParams p, double* __restrict__ out) {
   const int l = blockIdx.x;
   const int kl = p.sp_of[l];
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  const int ni = 2 * p.iesr + 1, nimg = ni * ni * ni;
-  for (int e = blockIdx.y * kThreads + threadIdx.x; e < p.nat * nimg; e += gridDim.y * kThreads) {
-    const int img = e / p.nat, m = e - img * p.nat;
-    const int ix = img / (ni * ni) - p.iesr, iy = img / ni % ni - p.iesr, iz = img % ni - p.iesr;
+  const int ni = 2 * p.iesr + 1;
+  const int dz = SHARES ? p.nz : 1;
+  int m0 = threadIdx.x, cc = 0, cz = 0;
+  if constexpr (SHARES) {   // below kThreads atoms a workgroup takes several shares of every partner
+    const int per = max(1, kThreads / p.nat), own = per > 1 ? threadIdx.x / p.nat : 0;
+    const int c = blockIdx.y * per + own;
+    m0 = own < per && c < p.ncol * p.nz ? threadIdx.x - own * p.nat : p.nat;
+    cc = c % p.ncol;
+    cz = c / p.ncol;
+  }
+  for (int m = m0; m < p.nat; m += kThreads) {
     const int km = p.sp_of[m];
     const double zv2 = p.zv[kl] * p.zv[km];
     if (fabs(zv2) < 1e-10) continue;
@@ -438,20 +451,32 @@ __global__ __launch_bounds__(kThreads) void k_ewald(EParams p, double* __restric
       for (int i = 0; i < 3; ++i) fr[i] -= nearbyint(fr[i]);
       for (int q = 0; q < 3; ++q) d[q] = fr[0] * p.a[q] + fr[1] * p.a[3 + q] + fr[2] * p.a[6 + q];
     }
-    if (tzero && ix == 0 && iy == 0 && iz == 0) continue;
-    double r[3];
-    for (int q = 0; q < 3; ++q) r[q] = d[q] + ix * p.a[q] + iy * p.a[3 + q] + iz * p.a[6 + q];
-    const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-    const double rl = sqrt(r2);
-    const double arg = rl / rckj;
-    if (arg > 20.0) continue;
-    const double add = zv2 * erfc(arg) / rl;
-    acc[0] += 0.5 * add;
-    if (!tzero) {
-      const double rep = (add + 2.0 * zv2 / sqrt(M_PI) * exp(-arg * arg) / rckj) / r2;
-      acc[1] += rep * r[0];
-      acc[2] += rep * r[1];
-      acc[3] += rep * r[2];
+    const auto column = [&](int ix, int iy) {
+      double b[3];
+      for (int q = 0; q < 3; ++q) b[q] = d[q] + ix * p.a[q] + iy * p.a[3 + q];
+      for (int iz = cz - p.iesr; iz <= p.iesr; iz += dz) {
+        if (tzero && ix == 0 && iy == 0 && iz == 0) continue;
+        double r[3];
+        for (int q = 0; q < 3; ++q) r[q] = b[q] + iz * p.a[6 + q];
+        const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+        const double rl = sqrt(r2);
+        const double arg = rl / rckj;
+        if (arg > 20.0) continue;
+        const double add = zv2 * erfc(arg) / rl;
+        acc[0] += 0.5 * add;
+        if (!tzero) {
+          const double rep = (add + 2.0 * zv2 / sqrt(M_PI) * exp(-arg * arg) / rckj) / r2;
+          acc[1] += rep * r[0];
+          acc[2] += rep * r[1];
+          acc[3] += rep * r[2];
+        }
+      }
+    };
+    if constexpr (SHARES) {
+      for (int xy = cc; xy < ni * ni; xy += p.ncol) column(xy / ni - p.iesr, xy % ni - p.iesr);
+    } else {
+      for (int ix = -p.iesr; ix <= p.iesr; ++ix)
+        for (int iy = -p.iesr; iy <= p.iesr; ++iy) column(ix, iy);
     }
   }
   block_sum_store<4>(acc, out + 4 * ((size_t)blockIdx.y * p.nat + l), 4);
@@ -880,11 +905,18 @@ void ewald(mc_ctx* ctx, int iesr, double* esr, double* eself, double* fion_host)
   p.sp_of = D.d_sp_of.as<int>();
   p.zv = D.d_zv.as<double>();
   p.raggio = D.d_raggio.as<double>();
-  // workgroups per atom: enough for the chip, each with several passes of its threads
-  const long long pairs = (long long)nat * (2 * iesr + 1) * (2 * iesr + 1) * (2 * iesr + 1);
-  const int ny = (int)std::max(1LL, std::min<long long>((2048 + nat - 1) / nat, pairs / (2 * kThreads)));
+  // a thread per partner where that fills the chip (512 workgroups of 256); below,
+  // the images of a partner go to several threads
+  const long long want = 512LL * kThreads / ((long long)nat * nat);
+  const int ni = 2 * iesr + 1;
+  p.ncol = (int)std::max(1LL, std::min<long long>(ni * ni, want));
+  p.nz = (int)std::max(1LL, std::min<long long>(ni, want / p.ncol));
+  const int per = std::max(1, kThreads / nat), ny = (p.ncol * p.nz + per - 1) / per;
   D.w_part.ensure(sizeof(double) * 4 * (size_t)nat * ny);
-  LAUNCH(MC_KID_VOFRHO, k_ewald, dim3(nat, ny), dim3(kThreads), 0, p, D.w_part.as<double>());
+  if (p.ncol * p.nz > 1)
+    LAUNCH(MC_KID_VOFRHO, k_ewald<true>, dim3(nat, ny), dim3(kThreads), 0, p, D.w_part.as<double>());
+  else
+    LAUNCH(MC_KID_VOFRHO, k_ewald<false>, dim3(nat), dim3(kThreads), 0, p, D.w_part.as<double>());
   std::vector<double> h(4 * (size_t)nat * ny);
   dl_add(ctx, h.data(), D.w_part.p, sizeof(double) * h.size());
   dl_finish(ctx);
