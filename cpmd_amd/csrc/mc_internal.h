@@ -225,11 +225,10 @@ struct DensitySet {
   std::vector<int> na;
   std::vector<double> zv, raggio, tau;
   double a[9] = {}, inv[9] = {};   // lattice vectors a[3i+q]; fractional f_i = sum_q d_q inv[3q+i]
-  DevBuf d_gm, d_gidx, d_scg, d_gk;
+  DevBuf d_perm, d_gm3, d_gidx, d_scg, d_gk;   // d_perm: device order of the G's -> the caller's (vofrho.hip)
   DevBuf d_sp_start, d_sp_of, d_zv, d_raggio, d_vps, d_rhops;
   DevBuf d_tau, d_ph1, d_ph2, d_ph3;   // d_tau: [tau (3, nat) | fractional coordinates (3, nat)]
   DevBuf w_W, w_V, w_part;
-  std::vector<int> gperm;   // device order of the G's -> the caller's (vofrho.hip)
   // z-sticks of the density set: the distinct (m1, m2) (d_stk, m1 fastest) and
   // the stick of each G (d_sidx); G_k = base_k(stick) + m3 b3_k (nby = 2); operands
   // of the stick GEMMs of vofrho

@@ -30,6 +30,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <memory>
 #include <vector>
 
 #include "fft_launch.h"
@@ -220,21 +221,17 @@ __global__ void k_phase_tables(const double* __restrict__ frac, int nat, int n1,
 }
 
 struct GParams {
-  int nhg, geq0, nsp, nat;
-  int h1, h2, h3;            // n_k / 2
-  const int* gm;             // (3, nhg) centred indices m
+  int nhg, geq0, nsp;
+  int h3;                    // n3 / 2
+  const int* gm3;            // (nhg) centred index m3
   const int* gidx;           // (2, nhg) linear W index of +G, -G
   const double* scg;         // (nhg)
   const double* vps;         // (nsp, nhg)
   const double* rhops;       // (nsp, nhg)
-  const int* sp_start;       // (nsp + 1) first atom of each species
-  const double2* ph1;
-  const double2* ph2;
-  const double2* ph3;
   const int* sidx;           // (nhg) stick of each G
-  int nstick, lds, L3;       // sticks, their even leading dimension; L3 = n3 + 1 positions m3 + h3 per stick
+  int lds, L3;               // the sticks' even leading dimension; L3 = n3 + 1 positions m3 + h3 per stick
   const double* sf;          // (nsp) blocks of (lds x 2 L3): Re | Im of the structure factor
-  const double* gk;          // (3, nhg)
+  const double* gk;          // (3, nhg), set if nby = 3
   int nby;                   // stick operand of potfor: 2 blocks (X, X m3) or 3 (X G_k)
 };
 
@@ -257,7 +254,7 @@ __global__ __launch_bounds__(kThreads) void k_eicalc_ppener(GParams g, const dou
     const double2 w = W[ip];
     const double2 re = make_double2(w.x * scale, w.y * scale);
     double2 ev = make_double2(0.0, 0.0), er = make_double2(0.0, 0.0);
-    const int m3 = g.gm[3 * ig + 2], st = g.sidx[ig];
+    const int m3 = g.gm3[ig], st = g.sidx[ig];
     const size_t ps = (size_t)(m3 + g.h3) * g.lds + st;
     for (int is = 0; is < g.nsp; ++is) {
       const double* S = g.sf + (size_t)is * g.lds * 2 * g.L3;
@@ -502,35 +499,53 @@ __global__ void k_eigr(const int* __restrict__ gmw, int ngw, int ldg, int n1, in
 // ---------------------------------------------------------------------------
 // host drivers
 // ---------------------------------------------------------------------------
+// dst(is, j) = src(is, perm[j])
+__global__ void k_gather_g(const double* __restrict__ src, const int* __restrict__ perm, int nsp, int nhg,
+                           double* __restrict__ dst) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= nhg) return;
+  for (int is = 0; is < nsp; ++is) dst[is + (size_t)nsp * j] = src[is + (size_t)nsp * perm[j]];
+}
+
 void set_density_gset(mc_ctx* ctx, int nhg, const int* inyh, const double* hg, const double* gk) {
   auto& D = ctx->dens;
   MC_CHECK(nhg >= 1, MC_ERR_ARG, "set_density_gset: nhg < 1");
   const int nr[3] = {ctx->n1, ctx->n2, ctx->n3};
-  for (int ig = 0; ig < nhg; ++ig)
-    for (int k = 0; k < 3; ++k) {
-      const int m = inyh[3 * (size_t)ig + k] - (nr[k] / 2 + 1);
-      MC_CHECK(m >= -nr[k] / 2 && m <= nr[k] / 2, MC_ERR_ARG, "set_density_gset: G index outside the mesh");
-      if (ig == 0 && ctx->geq0) MC_CHECK(m == 0, MC_ERR_ARG, "set_density_gset: first G must be G = 0");
-    }
-  // device order: G = 0 first (geq0), then m1 fastest, m2, m3 (two stable counting
-  // sorts)
   const int first = ctx->geq0 ? 1 : 0;
-  std::vector<int> perm(nhg), tmp(nhg);
-  for (int ig = 0; ig < nhg; ++ig) perm[ig] = ig;
-  const auto sort_by = [&](auto key, int nkey) {
-    std::vector<int> pos(nkey + 1, 0);
-    for (int j = first; j < nhg; ++j) ++pos[key(perm[j]) + 1];
-    for (int v = 0; v < nkey; ++v) pos[v + 1] += pos[v];
-    for (int j = first; j < nhg; ++j) tmp[first + pos[key(perm[j])]++] = perm[j];
-    perm.swap(tmp);
-    if (first) perm[0] = 0;
+  // device order: G = 0 first (geq0), then m1 fastest, m2, m3 (two stable counting
+  // sorts, of i1 and of the row i2 + w2 i3).  The arrays are written before they are
+  // read: no zeros first, the pages alone cost as much as a sort.
+  const auto room = [](auto v, size_t n) { return std::unique_ptr<decltype(v)[]>(new decltype(v)[n]); };
+  const int w1 = nr[0] + 2, w2 = nr[1] + 2, nrow = w2 * (nr[2] + 2);
+  std::vector<int> end1(w1 + 1, 0), end2(nrow + 1, 0), sid((size_t)w1 * w2, -1);
+  for (int ig = 0; ig < nhg; ++ig) {
+    const int* i = inyh + 3 * (size_t)ig;
+    for (int k = 0; k < 3; ++k) {
+      const int m = i[k] - (nr[k] / 2 + 1);
+      MC_CHECK(m >= -nr[k] / 2 && m <= nr[k] / 2, MC_ERR_ARG, "set_density_gset: G index outside the mesh");
+      if (ig < first) MC_CHECK(m == 0, MC_ERR_ARG, "set_density_gset: first G must be G = 0");
+    }
+    if (ig >= first) {
+      MC_CHECK(hg[ig] > 0.0, MC_ERR_ARG, "set_density_gset: G = 0 after the first position");
+      ++end1[i[0] + 1];
+      ++end2[i[1] + w2 * i[2] + 1];
+    }
+    sid[i[0] + (size_t)w1 * i[1]] = 0;
+  }
+  for (int v = 0; v < w1; ++v) end1[v + 1] += end1[v];   // [v]: start of bin v, its end once filled
+  for (int v = 0; v < nrow; ++v) end2[v + 1] += end2[v];
+  struct Rec {
+    int ig, key;
   };
-  const int w1 = nr[0] + 2, w2 = nr[1] + 2;
-  sort_by([&](int ig) { return inyh[3 * (size_t)ig]; }, w1);
-  sort_by([&](int ig) { return inyh[3 * (size_t)ig + 1] + w2 * inyh[3 * (size_t)ig + 2]; }, w2 * (nr[2] + 2));
-  // z-sticks: the distinct (m1, m2) in the order (m2, m1), and the stick of each G
-  std::vector<int> sid((size_t)w1 * w2, -1);
-  for (int ig = 0; ig < nhg; ++ig) sid[inyh[3 * (size_t)ig] + (size_t)w1 * inyh[3 * (size_t)ig + 1]] = 0;
+  const int nsort = nhg - first;
+  const auto by1 = room(Rec{}, nsort), by2 = room(Rec{}, nsort);
+  for (int ig = first; ig < nhg; ++ig) {
+    const int* i = inyh + 3 * (size_t)ig;
+    by1[end1[i[0]]++] = Rec{ig, i[1] + w2 * i[2]};
+  }
+  for (int v = 0, e = 0; v < w1; ++v)
+    for (; e < end1[v]; ++e) by2[end2[by1[e].key]++] = Rec{by1[e].ig, v};
+  // z-sticks: the distinct (m1, m2) in the order (m2, m1)
   int nstick = 0;
   std::vector<int> stk;
   for (size_t e = 0; e < sid.size(); ++e)
@@ -539,72 +554,73 @@ void set_density_gset(mc_ctx* ctx, int nhg, const int* inyh, const double* hg, c
       stk.push_back((int)(e % w1) - (nr[0] / 2 + 1));
       stk.push_back((int)(e / w1) - (nr[1] / 2 + 1));
     }
-  std::vector<int> gm((size_t)3 * nhg), gidx((size_t)2 * nhg), sidx(nhg);
-  std::vector<double> scg(nhg), gks((size_t)3 * nhg);
-  for (int j = 0; j < nhg; ++j) {
-    const size_t ig = perm[j];
+  const auto perm = room(0, nhg), gm3 = room(0, nhg), gidx = room(0, 2 * (size_t)nhg), sidx = room(0, nhg);
+  const auto scg = room(0.0, nhg);
+  const auto place = [&](int j, int ig, int i1, int i2, int i3) {
+    const int m[3] = {i1 - (nr[0] / 2 + 1), i2 - (nr[1] / 2 + 1), i3 - (nr[2] / 2 + 1)};
     int ip[3], im[3];
     for (int k = 0; k < 3; ++k) {
-      const int m = inyh[3 * ig + k] - (nr[k] / 2 + 1);
-      gm[3 * (size_t)j + k] = m;
-      ip[k] = m < 0 ? m + nr[k] : m % nr[k];
-      im[k] = m > 0 ? nr[k] - m : -m % nr[k];
-      gks[3 * (size_t)j + k] = gk[3 * ig + k];
+      ip[k] = m[k] < 0 ? m[k] + nr[k] : m[k] % nr[k];
+      im[k] = m[k] > 0 ? nr[k] - m[k] : -m[k] % nr[k];
     }
+    perm[j] = ig;
+    gm3[j] = m[2];
     gidx[2 * (size_t)j] = ip[0] + nr[0] * (ip[1] + nr[1] * ip[2]);
     gidx[2 * (size_t)j + 1] = im[0] + nr[0] * (im[1] + nr[1] * im[2]);
-    sidx[j] = sid[inyh[3 * ig] + (size_t)w1 * inyh[3 * ig + 1]];
-    if (j == 0 && ctx->geq0) {
-      scg[j] = 0.0;
-    } else {
-      MC_CHECK(hg[ig] > 0.0, MC_ERR_ARG, "set_density_gset: G = 0 after the first position");
-      scg[j] = 4.0 * M_PI / (ctx->tpiba2 * hg[ig]);
-    }
-  }
+    sidx[j] = sid[i1 + (size_t)w1 * i2];
+    scg[j] = j < first ? 0.0 : 4.0 * M_PI / (ctx->tpiba2 * hg[ig]);
+  };
+  if (first) place(0, 0, inyh[0], inyh[1], inyh[2]);
+  for (int v = 0, e = 0; v < nrow; ++v)
+    for (; e < end2[v]; ++e) place(e + first, by2[e].ig, by2[e].key, v % w2, v / w2);
   // G_k = base_k(stick) + m3 b3_k: b3 from the stick with the widest range of m3,
-  // base from the first G of each stick; nby = 3 when the set does not fit that
+  // base from the lowest G of each stick; nby = 3 when the set does not fit that
+  const auto stick = [&](int ig) { return sid[inyh[3 * (size_t)ig] + (size_t)w1 * inyh[3 * (size_t)ig + 1]]; };
+  const auto at = [&](int ig) { return inyh[3 * (size_t)ig + 2] - (nr[2] / 2 + 1); };   // m3
   std::vector<int> lo(nstick, -1), hi(nstick, -1);
-  for (int j = 0; j < nhg; ++j) {   // m3 rises with j behind G = 0
-    const int st = sidx[j];
-    if (lo[st] < 0 || gm[3 * (size_t)j + 2] < gm[3 * (size_t)lo[st] + 2]) lo[st] = j;
-    if (hi[st] < 0 || gm[3 * (size_t)j + 2] > gm[3 * (size_t)hi[st] + 2]) hi[st] = j;
+  double gmax = 0.0;
+  for (int ig = 0; ig < nhg; ++ig) {
+    const int st = stick(ig), m = at(ig);
+    if (lo[st] < 0 || m < at(lo[st])) lo[st] = ig;
+    if (hi[st] < 0 || m > at(hi[st])) hi[st] = ig;
+    for (int k = 0; k < 3; ++k) gmax = std::max(gmax, std::fabs(gk[3 * (size_t)ig + k]));
   }
   int wide = 0, span = -1;
-  for (int st = 0; st < nstick; ++st) {
-    const int d = gm[3 * (size_t)hi[st] + 2] - gm[3 * (size_t)lo[st] + 2];
-    if (d > span) {
-      span = d;
+  for (int st = 0; st < nstick; ++st)
+    if (at(hi[st]) - at(lo[st]) > span) {
+      span = at(hi[st]) - at(lo[st]);
       wide = st;
     }
-  }
   std::vector<double> base((size_t)3 * nstick);
-  double gmax = 0.0;
   for (int k = 0; k < 3; ++k)
-    D.b3[k] = span > 0 ? (gks[3 * (size_t)hi[wide] + k] - gks[3 * (size_t)lo[wide] + k]) / span : 0.0;
+    D.b3[k] = span > 0 ? (gk[3 * (size_t)hi[wide] + k] - gk[3 * (size_t)lo[wide] + k]) / span : 0.0;
   for (int st = 0; st < nstick; ++st)
-    for (int k = 0; k < 3; ++k)
-      base[3 * (size_t)st + k] = gks[3 * (size_t)lo[st] + k] - gm[3 * (size_t)lo[st] + 2] * D.b3[k];
-  for (double x : gks) gmax = std::max(gmax, std::fabs(x));
+    for (int k = 0; k < 3; ++k) base[3 * (size_t)st + k] = gk[3 * (size_t)lo[st] + k] - at(lo[st]) * D.b3[k];
   D.nby = 2;
-  for (int j = 0; j < nhg && D.nby == 2; ++j)
+  for (int ig = 0; ig < nhg && D.nby == 2; ++ig) {
+    const double* b = base.data() + 3 * (size_t)stick(ig);
     for (int k = 0; k < 3; ++k)
-      if (!(std::fabs(base[3 * (size_t)sidx[j] + k] + gm[3 * (size_t)j + 2] * D.b3[k] - gks[3 * (size_t)j + k]) <=
-            1e-14 * gmax))
-        D.nby = 3;
+      if (!(std::fabs(b[k] + at(ig) * D.b3[k] - gk[3 * (size_t)ig + k]) <= 1e-14 * gmax)) D.nby = 3;
+  }
   D.nstick = nstick;
   D.nhg = nhg;
-  D.gperm = perm;
   const auto put = [](DevBuf& b, const void* p, size_t bytes) {
     b.ensure(bytes);
     MC_HIP(hipMemcpy(b.p, p, bytes, hipMemcpyHostToDevice));
   };
-  put(D.d_sidx, sidx.data(), sizeof(int) * sidx.size());
+  put(D.d_perm, perm.get(), sizeof(int) * (size_t)nhg);
+  put(D.d_sidx, sidx.get(), sizeof(int) * (size_t)nhg);
   put(D.d_stk, stk.data(), sizeof(int) * stk.size());
   put(D.d_base, base.data(), sizeof(double) * base.size());
-  put(D.d_gm, gm.data(), sizeof(int) * gm.size());
-  put(D.d_gidx, gidx.data(), sizeof(int) * gidx.size());
-  put(D.d_scg, scg.data(), sizeof(double) * scg.size());
-  put(D.d_gk, gks.data(), sizeof(double) * gks.size());
+  put(D.d_gm3, gm3.get(), sizeof(int) * (size_t)nhg);
+  put(D.d_gidx, gidx.get(), sizeof(int) * 2 * (size_t)nhg);
+  put(D.d_scg, scg.get(), sizeof(double) * (size_t)nhg);
+  if (D.nby == 3) {
+    const auto gks = room(0.0, 3 * (size_t)nhg);
+    for (int j = 0; j < nhg; ++j)
+      for (int k = 0; k < 3; ++k) gks[3 * (size_t)j + k] = gk[3 * (size_t)perm[j] + k];
+    put(D.d_gk, gks.get(), sizeof(double) * 3 * (size_t)nhg);
+  }
   D.ready = true;
   D.pp_ready = false;
 }
@@ -638,14 +654,16 @@ void set_local_pp(mc_ctx* ctx, int nsp, const int* na, const double* zv, const d
   MC_HIP(hipMemcpy(D.d_sp_of.p, sp_of.data(), sizeof(int) * sp_of.size(), hipMemcpyHostToDevice));
   MC_HIP(hipMemcpy(D.d_zv.p, zv, sizeof(double) * nsp, hipMemcpyHostToDevice));
   MC_HIP(hipMemcpy(D.d_raggio.p, raggio, sizeof(double) * nsp, hipMemcpyHostToDevice));
-  // in the device order of the G's
-  std::vector<double> x((size_t)nsp * D.nhg);
+  // into the device order of the G's, the caller's order passing through the mesh
+  // buffer of vofrho
+  const size_t bytes = sizeof(double) * (size_t)nsp * D.nhg;
+  D.w_V.ensure(bytes);
   for (int w = 0; w < 2; ++w) {
-    const double* src = w ? rhops : vps;
-    for (int j = 0; j < D.nhg; ++j)
-      for (int is = 0; is < nsp; ++is) x[is + (size_t)nsp * j] = src[is + (size_t)nsp * D.gperm[j]];
-    MC_HIP(hipMemcpy((w ? D.d_rhops : D.d_vps).p, x.data(), sizeof(double) * x.size(), hipMemcpyHostToDevice));
+    MC_HIP(hipMemcpyAsync(D.w_V.p, w ? rhops : vps, bytes, hipMemcpyHostToDevice, ctx->stream));
+    LAUNCH(MC_KID_MISC, k_gather_g, dim3((D.nhg + 255) / 256), dim3(256), 0, D.w_V.as<double>(), D.d_perm.as<int>(),
+           nsp, D.nhg, (w ? D.d_rhops : D.d_vps).as<double>());
   }
+  MC_HIP(hipStreamSynchronize(ctx->stream));
   D.pp_ready = true;
   D.ions_ready = false;
 }
@@ -711,21 +729,13 @@ static GParams make_gparams(mc_ctx* ctx) {
   g.nhg = D.nhg;
   g.geq0 = ctx->geq0;
   g.nsp = D.nsp;
-  g.nat = D.nat;
-  g.h1 = ctx->n1 / 2;
-  g.h2 = ctx->n2 / 2;
   g.h3 = ctx->n3 / 2;
-  g.gm = D.d_gm.as<int>();
+  g.gm3 = D.d_gm3.as<int>();
   g.gidx = D.d_gidx.as<int>();
   g.scg = D.d_scg.as<double>();
   g.vps = D.d_vps.as<double>();
   g.rhops = D.d_rhops.as<double>();
-  g.sp_start = D.d_sp_start.as<int>();
-  g.ph1 = D.d_ph1.as<double2>();
-  g.ph2 = D.d_ph2.as<double2>();
-  g.ph3 = D.d_ph3.as<double2>();
   g.sidx = D.d_sidx.as<int>();
-  g.nstick = D.nstick;
   g.lds = D.nstick + (D.nstick & 1);
   g.gk = D.d_gk.as<double>();
   g.nby = D.nby;
@@ -787,7 +797,8 @@ void vofrho_dev(mc_ctx* ctx, const double* rho, double* v, double* energies, dou
   if (nat > 0) {
     const int nqb = (ls + 255) / 256;
     LAUNCH(MC_KID_VOFRHO, k_stick_ops, dim3(nqb + (L3 + 255) / 256, nat), dim3(256), 0, D.d_stk.as<int>(), ns, ls,
-           ctx->n1, ctx->n2, ctx->n3, nat, nqb, g.ph1, g.ph2, g.ph3, D.d_sp_of.as<int>(), D.d_sp_start.as<int>(), Q,
+           ctx->n1, ctx->n2, ctx->n3, nat, nqb, D.d_ph1.as<double2>(), D.d_ph2.as<double2>(),
+           D.d_ph3.as<double2>(), D.d_sp_of.as<int>(), D.d_sp_start.as<int>(), Q,
            D.w_bs.as<double>(), D.w_bf.as<double>());
   }
   {
