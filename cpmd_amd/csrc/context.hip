@@ -141,6 +141,20 @@ size_t mem_current() {
   return mem().cur;
 }
 
+bool try_ensure(DevBuf& b, size_t bytes, bool must) {
+  if (must) {
+    b.ensure(bytes);
+    return true;
+  }
+  try {
+    b.ensure(bytes);
+  } catch (const Error&) {
+    (void)hipGetLastError();   // a failed hipMalloc leaves its error behind
+    return false;
+  }
+  return true;
+}
+
 void DevBuf::ensure(size_t nbytes) {
   if (nbytes <= bytes) return;
   release();

@@ -527,9 +527,11 @@ bool tn_f64_form(const double* A, int lda, const double* B, int ldb) {
 }
 
 // Partials of A^T B into ctx->w_gemm; returns their number.  proj: A is the
-// projector operand of m columns (A, lda unused).
+// projector operand of m columns (A, lda unused).  Where the device memory does not
+// hold the partials, K is split less (with fewer); where it still does not, an error,
+// or 0 for the projector operand.
 int tn_f64_partials(mc_ctx* ctx, const double* A, int lda, const double* B, int ldb, int K, int m, int n,
-                    bool symmetric, const ProjTab* proj) {
+                    bool symmetric, const ProjTab* proj, bool fewer) {
   const int mu = proj ? proj->ncol : m;   // rows that decide the tile and the split
   int ni = 2, nj = 1;
   if (symmetric) {   // square tiles
@@ -570,10 +572,15 @@ int tn_f64_partials(mc_ctx* ctx, const double* A, int lda, const double* B, int 
       nsplit = s;
     }
   }
-  int kchunk = (K + nsplit - 1) / nsplit;
-  kchunk = (kchunk + kKs - 1) / kKs * kKs;
-  nsplit = (K + kchunk - 1) / kchunk;
-  ctx->w_gemm.ensure(sizeof(double) * (size_t)nsplit * m * n);
+  int kchunk;
+  for (;; nsplit /= 2) {
+    kchunk = (K + nsplit - 1) / nsplit;
+    kchunk = (kchunk + kKs - 1) / kKs * kKs;
+    nsplit = (K + kchunk - 1) / kchunk;
+    const bool last = nsplit == 1 || !fewer;
+    if (try_ensure(ctx->w_gemm, sizeof(double) * (size_t)nsplit * m * n, last && !proj)) break;
+    if (last) return 0;
+  }
   const int total = nsplit * tiles;
   timer_begin(ctx, MC_KID_GEMM_TN);
   if (ni == 2)

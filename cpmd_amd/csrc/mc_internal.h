@@ -100,6 +100,10 @@ struct DevBuf {
   T* as() const { return static_cast<T*>(p); }
 };
 
+// b.ensure(bytes) where the device memory (its limit) holds them; otherwise false, b
+// then being empty, or the error with `must`.
+bool try_ensure(DevBuf& b, size_t bytes, bool must = false);
+
 // Reclaimable workspaces (the transform batch buffers of every context).  An
 // allocation that would take the library beyond the device memory limit first
 // frees the registered workspaces that no call is using, then tries again;
@@ -418,7 +422,7 @@ void reduce_tn_rows(mc_ctx* ctx, int nsplit, int ldp, int r0, int m, int n, doub
 // FP64 products of aligned operands (gemm_f64.hip)
 bool tn_f64_form(const double* A, int lda, const double* B, int ldb);
 int tn_f64_partials(mc_ctx* ctx, const double* A, int lda, const double* B, int ldb, int K, int m, int n,
-                    bool symmetric, const ProjTab* proj);
+                    bool symmetric, const ProjTab* proj, bool fewer = true);
 bool nn_f64_form(const double* A, int lda, int M, const double* D, int ldd, const FnlEpi* epi);
 void nn_f64(mc_ctx* ctx, const double* A, int lda, const double* G, int ldgm, int M, int k, int n, double alpha,
             double beta, double* D, int ldd, bool upper_g, const FnlEpi& epi, const ProjTab* proj, int kid);

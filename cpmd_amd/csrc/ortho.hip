@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <functional>
 #include <vector>
 
 #include "mc_internal.h"
@@ -609,10 +610,27 @@ static void rnlsm_groups(mc_ctx* ctx, const double2* c0, int n, bool do_fnl, boo
   const int ldf = P.nat * P.nhxs, ldd = P.nat * P.nhxs * 3;
   const bool stacked = !x3 && tn_f64_form(B, ldb, B, ldb);
   if (stacked && P.ncol > 0 && n > 0) {
-    const ProjTab t = proj_tab(ctx, do_fnl ? 0 : 1);
-    const int nv = (do_fnl ? 1 : 0) + (do_dfnl ? 3 : 0);
-    const int ns = tn_f64_partials(ctx, nullptr, 0, B, ldb, K, nv * P.ncol, n, false, &t);
-    reduce_proj(ctx, ns, t, nv, n, P.nat, P.nhxs, tpiba, P.d_fnl.as<double>(), P.d_dfnl.as<double>());
+    // nv variants from v0 of the nc columns from c0.  Where the device memory does
+    // not hold the partials of all, first single variants (the same bits), then
+    // fewer splits of K, then half the columns
+    const std::function<void(int, int, int, int)> run = [&](int v0, int nv, int c0, int nc) {
+      ProjTab t = proj_tab(ctx, v0);
+      t.tab += c0;
+      t.ncol = nc;
+      const int ns = tn_f64_partials(ctx, nullptr, 0, B, ldb, K, nv * nc, n, false, &t, nv == 1);
+      if (ns == 0) {
+        MC_CHECK(nv * nc > 1, MC_ERR_ARG, "rnlsm: the device memory limit leaves no room for one projector's sums");
+        if (nv > 1) {
+          for (int v = 0; v < nv; ++v) run(v0 + v, 1, c0, nc);
+        } else {
+          run(v0, 1, c0, nc / 2);
+          run(v0, 1, c0 + nc / 2, nc - nc / 2);
+        }
+        return;
+      }
+      reduce_proj(ctx, ns, t, nv, n, P.nat, P.nhxs, tpiba, P.d_fnl.as<double>(), P.d_dfnl.as<double>());
+    };
+    run(do_fnl ? 0 : 1, (do_fnl ? 1 : 0) + (do_dfnl ? 3 : 0), 0, P.ncol);
   }
   int isa0 = 0;
   for (int is = 0; is < P.nsp && !stacked; ++is) {
@@ -783,14 +801,14 @@ void fnonloc_dev(mc_ctx* ctx, double2* c2, const double* f_host, int n, const do
   const int M = wfn_rows(ctx);
   int groups = 0;
   for (int is = 0; is < P.nsp; ++is) groups += P.na[is] > 0 ? P.ngh[is] : 0;
-  if (groups > 1 && !(ctx->gemm_x3 && M >= kX3Min) && nn_f64_form((const double*)c2, wfn_ld(ctx), M, (const double*)c2, wfn_ld(ctx), nullptr)) {
+  if (groups > 1 && !(ctx->gemm_x3 && M >= kX3Min) &&
+      nn_f64_form((const double*)c2, wfn_ld(ctx), M, (const double*)c2, wfn_ld(ctx), nullptr) &&
+      try_ensure(ctx->w_dd, sizeof(double) * (size_t)P.ncol * n)) {
     // one product over all projector columns: c2 is read and written once (64
     // atoms of two species, 5 projectors, 130 states at 128^3: 0.27 ms against
     // 1.26 ms for a product per projector).  A single group takes the plain
     // product below, its factor applied to the result: eigr is then copied to
     // LDS as it is (256 atoms, 512 states, 192^3: 2.06 against 2.58 ms)
-    if (P.ncol == 0) return;
-    ctx->w_dd.ensure(sizeof(double) * (size_t)P.ncol * n);
     hipLaunchKernelGGL(k_fnl_dd_all, dim3((P.ncol + 63) / 64, n), dim3(64), 0, ctx->stream, P.d_fnl.as<double>(),
                        P.nat, P.nhxs, P.tab(), P.ncol, P.d_h.as<double>(),
                        ctx->w_dd.as<double>());

@@ -157,14 +157,7 @@ template <typename T>
 static v2<T>* keep_columns(mc_ctx* ctx, int npairs) {
   if (!ctx->col_reuse || mem_limit() != 0 || npairs <= 0) return nullptr;
   const size_t bytes = sizeof(v2<T>) * (size_t)npairs * ctx->n3 * ctx->ncols * ctx->n2;
-  try {
-    ctx->w_keep.ensure(bytes);
-  } catch (const Error&) {
-    (void)hipGetLastError();   // a failed hipMalloc leaves its error behind
-    ctx->w_keep.release();
-    return nullptr;
-  }
-  return ctx->w_keep.as<v2<T>>();
+  return try_ensure(ctx->w_keep, bytes) ? ctx->w_keep.as<v2<T>>() : nullptr;
 }
 
 static void upload_f(mc_ctx* ctx, const double* f_host, int nstate) {
