@@ -36,12 +36,13 @@ __device__ __forceinline__ double lane_value(double v, int src) {
 // rows: one wave (lane = column) eliminates within the panel in registers, the
 // pivot row's entries taken lane by lane, and all waves update the rows behind
 // it.  The panel loop stays rolled: fully unrolled, the instructions alone took
-// 180 us to fetch (this one: 46).  A pivot that is not positive ends the
+// 180 us to fetch (this one: 46, and 12 with one panel).  A pivot that is not positive ends the
 // factorisation: *info = its order.
 __device__ void factor_block(double* T, double* Y, double* inv, int nb, int kb, double* __restrict__ S, int lds,
                              double* __restrict__ X, int ldx, int* info, int* bad) {
   constexpr int kP = 16;
   const int w = threadIdx.x >> 6, c = threadIdx.x & 63;
+  const int np = (nb + kP - 1) / kP * kP;   // the panels behind are those of the identity
   if (threadIdx.x == 0) *bad = 0;
   for (int e = threadIdx.x; e < kCb * kCb; e += 256) {
     const int r = e / kCb, cc = e & (kCb - 1);
@@ -49,7 +50,7 @@ __device__ void factor_block(double* T, double* Y, double* inv, int nb, int kb, 
   }
   __syncthreads();
 #pragma unroll 1
-  for (int r0 = 0; r0 < kCb; r0 += kP) {
+  for (int r0 = 0; r0 < np; r0 += kP) {
     if (w == 0) {
       double t[kP];
 #pragma unroll
@@ -72,7 +73,7 @@ __device__ void factor_block(double* T, double* Y, double* inv, int nb, int kb, 
 #pragma unroll
     for (int j = 0; j < kP; ++j) u[j] = T[(r0 + j) * kLd + c];
 #pragma unroll 1
-    for (int r = r0 + kP + w; r < kCb; r += 4) {
+    for (int r = r0 + kP + w; r < np; r += 4) {
       double a = T[r * kLd + c];
 #pragma unroll
       for (int j = 0; j < kP; ++j) a -= T[(r0 + j) * kLd + r] * u[j];
@@ -90,7 +91,7 @@ __device__ void factor_block(double* T, double* Y, double* inv, int nb, int kb, 
   }
   // X = U^-1 by columns, panels from the last: x_k = b_k / U_kk, b_r -= U_rk x_k
 #pragma unroll 1
-  for (int r0 = kCb - kP; r0 >= 0; r0 -= kP) {
+  for (int r0 = np - kP; r0 >= 0; r0 -= kP) {
     if (w == 0) {
       double t[kP], b[kP];
 #pragma unroll

@@ -1,4 +1,4 @@
-"""Orthonormalisation of sets whose overlap is far from the unit matrix (start
+"""Orthonormalisation (lowdin, rgs) of sets whose overlap is far from the unit matrix (start
 orbitals, large steps): S = P diag(w) P^T with a geometric spectrum from 1 / cond
 to 1, C = Q diag(sqrt w) P^T with orthonormal Q."""
 import numpy as np
@@ -52,3 +52,17 @@ def test_lowdin(gpu, sysm, n, cond):
     iters = ctx.lowdin_dev(d, n)
     assert iters <= 40
     assert np.abs(ctx.download(d, n) - ref).max() < _tol(sysm, n, cond)
+
+
+@pytest.mark.parametrize("n", [2, 16, 17, 33, 50, 65, 130, 200])
+def test_rgs(gpu, sysm, n):
+    """C U^-1 is the Q of C = Q R with a positive diagonal; n at the edges of the
+    16-row panels and 64-wide blocks of the factorisation."""
+    ctx = ops.Context(sysm.cell, sysm.gset)
+    c, _ = _set(sysm, n, 1e6, n)
+    x = np.zeros((2 * sysm.gset.ngw - 1, n))
+    x[0], x[1::2], x[2::2] = c[0].real, np.sqrt(2) * c[1:].real, np.sqrt(2) * c[1:].imag
+    q, r = np.linalg.qr(x)
+    g, smat = ctx.rgs(c)
+    assert np.abs(g - _pack(q * np.sign(np.diag(r)))).max() < _tol(sysm, n, 1e6)
+    assert not np.tril(smat, -1).any() and (np.diag(smat) > 0).all()
