@@ -2,10 +2,10 @@
 // (LAPACK dpotrf, upper) and X = U^-1 (dtrtri), in 64-wide blocks.
 //
 // The chain of dependent launches bounds it, so each does as much as it can: a
-// diagonal block is factored and inverted by one workgroup whose rows live in
-// registers (one barrier per column), the block row U_kj = X_kk^T S_kj uses that
-// inverse, and the launch that updates the trailing blocks also factors the next
-// diagonal one.  The off-diagonal blocks of X follow by doubling, X_12 = -X_11
+// diagonal block is factored and inverted by one workgroup in LDS, panels of 16 rows
+// in the registers of one wave (two barriers per panel), the block row U_kj = X_kk^T
+// S_kj uses that inverse, and the launch that updates the trailing blocks also factors
+// the next diagonal one.  The off-diagonal blocks of X follow by doubling, X_12 = -X_11
 // U_12 X_22.  128 states: 0.13 ms in 6 launches where an LDS element loop with
 // three barriers per column, forward substitution per column and one wavefront
 // per column of X took 0.31 ms.
@@ -36,8 +36,8 @@ __device__ __forceinline__ double lane_value(double v, int src) {
 // rows: one wave (lane = column) eliminates within the panel in registers, the
 // pivot row's entries taken lane by lane, and all waves update the rows behind
 // it.  The panel loop stays rolled: fully unrolled, the instructions alone took
-// 180 us to fetch (this one: 46, and 12 with one panel).  A pivot that is not positive ends the
-// factorisation: *info = its order.
+// 180 us to fetch (this one: 46, and 12 with one panel).  A pivot that is not positive
+// ends the factorisation: *info = its order.
 __device__ void factor_block(double* T, double* Y, double* inv, int nb, int kb, double* __restrict__ S, int lds,
                              double* __restrict__ X, int ldx, int* info, int* bad) {
   constexpr int kP = 16;
@@ -219,7 +219,9 @@ __global__ __launch_bounds__(256) void k_chol_update(double* __restrict__ S, int
   __shared__ double B[kCb * kLd];
   __shared__ double inv[kCb];
   __shared__ int bad;
-  if (*info) return;
+  // only the workgroup that may set *info looks at it: for the others it could change
+  // between two of their waves (what they form after a failure is not used)
+  if (blockIdx.x == 0 && *info) return;
   const int nt = (n - kb - 1) / kCb;   // block columns behind k
   int ti, tj;
   tile_ij(blockIdx.x, true, nt, nt, ti, tj);
@@ -253,8 +255,8 @@ __global__ __launch_bounds__(256) void k_chol_update(double* __restrict__ S, int
 }
 
 // One doubling step of X = U^-1 from blocks of s rows to 2 s: pair p covers the
-// rows o = 2 s p .. (first part s, second n2 <= s).  STEP 0: W_12 = U_12 X_22
-// into the lower half's mirror of W; STEP 1: X_12 = -X_11 W_12.  Workgroup (64
+// rows o = 2 s p .. (first part s, second n2 <= s).  STEP 0: W_12 = U_12 X_22,
+// at the place of U_12; STEP 1: X_12 = -X_11 W_12.  Workgroup (64
 // x 64 tile, pair); the triangular factor's zero blocks are skipped.
 template <int STEP>
 __global__ __launch_bounds__(256) void k_tri_double(const double* __restrict__ U, int ldu, int n, int s,
