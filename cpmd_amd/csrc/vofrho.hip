@@ -401,7 +401,7 @@ __global__ __launch_bounds__(kThreads) void k_stick_force(const double* __restri
 // of the images); the vector to m is reduced to the cell once per thread.  Bound by
 // FP64 arithmetic: erfc and exp where most images lie inside the cut-off, the
 // distance to the image where they do not.  The whole call with two images per
-// direction: 8 atoms 19 us, 256 45, 4096 2.85 ms; with one thread per partner at every
+// direction: 8 atoms 19 us, 256 43, 4096 2.85 ms; with one thread per partner at every
 // size 85, 49 and 2.85 (dealing single (image, partner) pairs, the vector formed anew
 // for each: 21, 88 and 11.1).
 // e_l = sum_m sum_images w zv_l zv_m erfc(r / rckj) / r with w = 1/2 (each
@@ -916,13 +916,13 @@ void ewald(mc_ctx* ctx, int iesr, double* esr, double* eself, double* fion_host)
   p.sp_of = D.d_sp_of.as<int>();
   p.zv = D.d_zv.as<double>();
   p.raggio = D.d_raggio.as<double>();
-  // a thread per partner where that fills the chip (512 workgroups of 256); below,
-  // the images of a partner go to several threads
-  const long long want = 512LL * kThreads / ((long long)nat * nat);
-  const int ni = 2 * iesr + 1;
-  p.ncol = (int)std::max(1LL, std::min<long long>(ni * ni, want));
-  p.nz = (int)std::max(1LL, std::min<long long>(ni, want / p.ncol));
-  const int per = std::max(1, kThreads / nat), ny = (p.ncol * p.nz + per - 1) / per;
+  // a thread per partner from 257 atoms on; below, the images of a partner go to
+  // several threads, in up to 512 workgroups: their sums are one copy of 16 KB (a
+  // larger one takes 8 us more: 40 atoms in 520 workgroups 30 us, in 360 22)
+  const int per = std::max(1, kThreads / nat), want = std::max(1, 512 / nat) * per, ni = 2 * iesr + 1;
+  p.ncol = std::min(ni * ni, want);
+  p.nz = std::min(ni, want / p.ncol);
+  const int ny = (p.ncol * p.nz + per - 1) / per;
   D.w_part.ensure(sizeof(double) * 4 * (size_t)nat * ny);
   if (p.ncol * p.nz > 1)
     LAUNCH(MC_KID_VOFRHO, k_ewald<true>, dim3(nat, ny), dim3(kThreads), 0, p, D.w_part.as<double>());
