@@ -15,7 +15,7 @@
 //    length-B DFT in registers.  Register DFTs of composite length recurse at
 //    compile time into radix 2/3/4/5/7 butterflies with exact constant twiddles
 //    (twiddle_consts.h).  Stage form (FP32 at the lengths of MC_MORE_SIZES): the
-//    stages of the runtime plan, grouped A and B points at a time in registers.
+//    stages of the runtime plan, grouped A and B <= 25 points at a time in registers.
 //  * fft_lines<T, DIR>: any 2^a 3^b 5^c 7^d length from a runtime plan: mixed-radix
 //    Stockham stages; stage s with radix R and p = product of previous radices
 //    maps butterfly i of a line to inputs x[i + q n/R], twiddles w^{q k n/(pR)}
@@ -311,8 +311,8 @@ MC_FAST_SHAPE(320, 16, 20)
 // edge, with factors A = 4 Q where the two stay close (band pruning).  The
 // runtime-plan engine divides by runtime lengths for every butterfly and passes
 // through LDS three to five times: density of 103 states on 108 x 120 x 160 in
-// FP64 0.65 against 3.69 ms, gradient of 61 states on 80 x 144 x 96 with FP32
-// transforms 0.33 against 1.08 ms.
+// FP64 0.58 against 3.69 ms, gradient of 61 states on 80 x 144 x 96 with FP32
+// transforms 0.36 against 1.08 ms.
 #define MC_FAST_SIZES(X) X(16) X(18) X(24) X(54) X(128) X(192) X(224) X(240)
 #define MC_MORE_SIZES(X)                                                                                    \
   X(30) X(32) X(36) X(40) X(48) X(60) X(64) X(72) X(80) X(90) X(96) X(100) X(108) X(120) X(144) X(150) X(160) \
@@ -350,8 +350,11 @@ constexpr int stage_split(int n) {
 // Which compile-time engine length N has: the four-step one (FP64, and FP32 at
 // the lengths of MC_FAST_SIZES) or, in FP32 at the others, the stages of the
 // runtime plan two groups at a time in registers (StockShape): the same
-// operations on the same values, so the results are those of the runtime plan
-// bit for bit.
+// operations on the same values in the same order.  Run beside the runtime plan's
+// kernels at each of these lengths on each axis, with and without pruning, vpsi had
+// the same bits everywhere, and rho those bits up to the last places of the FP64
+// charge sums that scale it.  That rests on which products the compiler fuses
+// (twmul_stage, stage_end) and can change with it: the tests hold FP32's 2e-6.
 template <typename T, int N>
 constexpr bool four_step() {
   if (sizeof(T) == 8) return true;

@@ -13,7 +13,7 @@
 // sticks in the order (m2, m1): neighbouring G's are neighbours on the mesh and
 // among the sticks, so that the per-G pass reads and writes whole lines (in
 // CPMD's order of |G|^2, i.e. scattered, three kernels took 325 us at 192^3 / 1.6M
-// G's, now one takes 48).
+// G's, now one takes 45).
 //
 // References: vofrhoa src/vofrhoa_utils.mod.F90:41-144 (fwfftn :92, potfor
 // :101, ppener :103-122), eicalc src/eicalc_utils.mod.F90:33-173, ppener
