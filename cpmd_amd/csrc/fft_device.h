@@ -349,7 +349,7 @@ constexpr int stage_split(int n) {
 
 // Which compile-time engine length N has: the four-step one (FP64, and FP32 at
 // the lengths of MC_FAST_SIZES) or, in FP32 at the others, the stages of the
-// runtime plan two groups at a time in registers (StockShape): the same
+// runtime plan two groups at a time in registers (stock_stages): the same
 // operations on the same values in the same order.  Run beside the runtime plan's
 // kernels at each of these lengths on each axis, with and without pruning, vpsi had
 // the same bits everywhere, and rho those bits up to the last places of the FP64

@@ -510,13 +510,14 @@ void set_projectors(mc_ctx* ctx, int nsp, const int* na, int nhxs, const int* ng
   P.h_h.assign(hmat, hmat + nh);
   // one upload: hmat and, behind it, the projector columns in (species,
   // projector, atom) order
-  MC_CHECK(nhxs < 0x8000, MC_ERR_ARG, "set_projectors: bad nhxs");
   std::vector<int4> tab;
-  for (int is = 0, isa0 = 0; is < nsp; isa0 += na[is++])
+  for (int is = 0, isa0 = 0; is < nsp; isa0 += na[is++]) {
+    MC_CHECK(ngh[is] < 0x8000, MC_ERR_ARG, "set_projectors: more than 32767 projectors of a species");   // 16 bits of tab
     for (int iv = 0; iv < ngh[is]; ++iv)
       for (int ia = 0; ia < na[is]; ++ia)
         tab.push_back(make_int4(isa0 + ia, is * nhxs + iv, ((lang[iv + (size_t)nhxs * is] % 4) + 4) % 4,
                                 iv | ngh[is] << 16));
+  }
   P.ncol = (int)tab.size();
   P.tab_off = (sizeof(double) * nh + 15) / 16 * 16;
   std::vector<char> up(P.tab_off + sizeof(int4) * tab.size());
